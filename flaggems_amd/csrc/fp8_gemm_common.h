@@ -199,12 +199,15 @@ __device__ __forceinline__ T* uniform_ptr(T* p) {
 
 // 16-byte accesses that other XCDs can see: written through to memory / read past this XCD's L2 (the same
 // cache-control bit the compiler sets for agent-scope atomic loads and stores).  Not tracked by the
-// compiler's wait-count insertion: callers wait explicitly.
+// compiler's wait-count insertion: callers wait explicitly.  The base may have come out of v_readfirstlane or v_readlane
+// (a spilled scalar) in the instruction before: a vector-memory instruction must not read a scalar register within five
+// wait states of a vector instruction that wrote it, and the compiler keeps that distance only for instructions of its
+// own, hence the s_nop.
 __device__ __forceinline__ void store_x4_agent(float* base, uint32_t byte_off, const v4f& v) {
-  asm volatile("global_store_dwordx4 %0, %1, %2 sc1" : : "v"(byte_off), "v"(v), "s"(base) : "memory");
+  asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1" : : "v"(byte_off), "v"(v), "s"(base) : "memory");
 }
 __device__ __forceinline__ void load_x4_agent(v4f& v, const float* base, uint32_t byte_off) {
-  asm volatile("global_load_dwordx4 %0, %1, %2 sc1" : "=v"(v) : "v"(byte_off), "s"(base) : "memory");
+  asm volatile("s_nop 4\n\tglobal_load_dwordx4 %0, %1, %2 sc1" : "=v"(v) : "v"(byte_off), "s"(base) : "memory");
 }
 
 
@@ -273,6 +276,10 @@ struct GroupedGemm {
   int64_t c_rows;
   const float* row_weight;
 };
+// Few rows per group, fp8_gemm_stream.hip: activation rows a pass of its kernel takes (16, 32 or 64), or 0 when the
+// problem is not one for it.
+int grouped_stream_rows(const GemmArgs& a, const GroupedGemm& grouped);
+int launch_grouped_stream(const GemmArgs& a, const GroupedGemm& grouped, int rows, void* workspace, size_t workspace_bytes, hipStream_t stream);
 int launch_grouped(const GemmArgs& a, const GroupedGemm& grouped, void* workspace, size_t workspace_bytes, hipStream_t stream);
 // workspace that lets launch_grouped read row-major activation scales from a transposed copy
 size_t grouped_workspace_bytes(int64_t M, int64_t K);
