@@ -1566,6 +1566,7 @@ int launch_grouped(const GemmArgs& g, const GroupedGemm& grouped, void* workspac
       FG_FAIL(FG_ERR_UNSUPPORTED, "grouped fp8 gemm: %lld gathered rows: the rows of A and of its scales must fit 32-bit byte offsets",
               (long long)grouped.x_rows);
   }
+  if (const int rows = grouped_stream_rows(g, grouped)) return launch_grouped_stream(g, grouped, rows, workspace, workspace_bytes, stream);
   return launch_block(g, kModeBlock, workspace, workspace_bytes, stream, &grouped);
 }
 
