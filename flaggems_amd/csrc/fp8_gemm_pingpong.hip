@@ -97,6 +97,9 @@ struct PpArgs {
   const int* groups;
   int n_groups;
   int64_t w_group_stride, ws_group_stride;
+  // Many groups: entry 1 + t holds (group, first row, end row) of tile row t, entry 0 the number of tile rows
+  // (group_tile_rows_kernel), and a walk that enters a tile reads one entry.  Null: it scans `groups` from the start.
+  const int4* tile_rows;
   // Grouped problem whose rows are gathered (row_index != nullptr): row m of the sorted order is row
   // row_index[m] / index_div of X and of its scales (the reference's MoE kernel reads its tokens the same way,
   // sorted_token_ids // top_k, src/flag_gems/fused/fused_moe.py:1111); entries are forced into [0, x_rows).
@@ -210,7 +213,11 @@ struct WalkT {
     }
     m0 = tm * TILE_ROWS; n0 = tn * kBN;
     m_end = a.g.M; group = 0;
-    if (GROUPED) {
+    if (GROUPED && a.tile_rows != nullptr) {
+      const int t = 1 + (tm < tiles_m ? tm : 0);
+      const auto* const entry = reinterpret_cast<const __attribute__((address_space(4))) int*>((uintptr_t)(a.tile_rows + t));
+      group = entry[0]; m0 = entry[1]; m_end = entry[2];
+    } else if (GROUPED) {
       // tile row tm of the whole problem -> segment and tile row inside it
       int begin = 0, t = tm, e = 0, end = 0;
       for (; e < a.n_groups; ++e) {
@@ -780,11 +787,15 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_pingpong_kernel(PpArgs a) {
 
   int n_tiles = a.n_tiles, tiles_m = g.tiles_m;
   if (GROUPED) {
-    tiles_m = 0;
-    for (int e = 0, begin = 0; e < a.n_groups; ++e) {
-      const int end = segment_end(a, e, begin);
-      tiles_m += (end - begin + kTileRows - 1) / kTileRows;
-      begin = end;
+    if (a.tile_rows != nullptr) {
+      tiles_m = *reinterpret_cast<const __attribute__((address_space(4))) int*>((uintptr_t)a.tile_rows);
+    } else {
+      tiles_m = 0;
+      for (int e = 0, begin = 0; e < a.n_groups; ++e) {
+        const int end = segment_end(a, e, begin);
+        tiles_m += (end - begin + kTileRows - 1) / kTileRows;
+        begin = end;
+      }
     }
     n_tiles = tiles_m * g.tiles_n;
     if (kCuts) {
@@ -1298,9 +1309,65 @@ bool transposition_pays(int64_t tiles, int64_t KB, int cus) {
 }
 size_t transposed_scales_bytes(int64_t M, int64_t KB) { return (size_t)((M * KB * 4 + 255) / 256 * 256); }
 
+// Tile rows of a grouped problem (PpArgs::tile_rows).  One block: the group ends, forced into ascending order and into
+// [0, M] as segment_end does, and the tile rows before every group by scans in LDS; then every tile row finds its group
+// by bisection.  Latency-bound, about 4 us; it pays from a few dozen groups on, because a walk that scans the table
+// costs about 0.1 us a group at every tile change of each of its three walkers (512 groups, 64 rows each, GEMM
+// [2048, 4096]: see launch_block).
+constexpr int kTableGroups = 2048;
+__global__ __launch_bounds__(1024) void group_tile_rows_kernel(const int* ends, int n_groups, int M, int tile_rows, int capacity, int4* out) {
+  __shared__ int s_end[kTableGroups], s_tiles[kTableGroups + 1], s_wave[2][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int e0 = 2 * tid, e1 = e0 + 1;
+  int v0 = e0 < n_groups ? ends[e0] : 0, v1 = e1 < n_groups ? ends[e1] : 0;
+  v0 = v0 < 0 ? 0 : (v0 < M ? v0 : M);
+  v1 = v1 < 0 ? 0 : (v1 < M ? v1 : M);
+  v1 = v1 > v0 ? v1 : v0;
+  int top = v1;  // running maximum
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(top, d);
+    if (lane >= d && o > top) top = o;
+  }
+  if (lane == 63) s_wave[0][wave] = top;
+  __syncthreads();
+  int before = __shfl_up(top, 1);
+  if (lane == 0) before = 0;
+  for (int w = 0; w < wave; ++w) before = s_wave[0][w] > before ? s_wave[0][w] : before;
+  v0 = v0 > before ? v0 : before;
+  v1 = v1 > v0 ? v1 : v0;
+  const int n0 = e0 < n_groups ? (v0 - before + tile_rows - 1) / tile_rows : 0;
+  const int n1 = e1 < n_groups ? (v1 - v0 + tile_rows - 1) / tile_rows : 0;
+  int sum = n0 + n1;
+  for (int d = 1; d < 64; d <<= 1) {
+    const int o = __shfl_up(sum, d);
+    if (lane >= d) sum += o;
+  }
+  if (lane == 63) s_wave[1][wave] = sum;
+  __syncthreads();
+  int tiles = sum - n0 - n1;
+  for (int w = 0; w < wave; ++w) tiles += s_wave[1][w];
+  s_end[e0] = v0; s_end[e1] = v1;
+  s_tiles[e0] = tiles; s_tiles[e1] = tiles + n0;
+  if (tid == 1023) s_tiles[kTableGroups] = tiles + n0 + n1;
+  __syncthreads();
+  const int all = s_tiles[n_groups] < capacity ? s_tiles[n_groups] : capacity;
+  if (tid == 0) out[0] = int4{all, 0, 0, 0};
+  for (int t = tid; t < all; t += 1024) {
+    int lo = 0, hi = n_groups - 1;  // the last group with at most t tile rows before it
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (s_tiles[mid] <= t) lo = mid; else hi = mid - 1;
+    }
+    const int begin = lo > 0 ? s_end[lo - 1] : 0;
+    out[1 + t] = int4{lo, begin + (t - s_tiles[lo]) * tile_rows, s_end[lo], 0};
+  }
+}
+
 // Short tiles of grouped problems (the JN = 1 instantiation) and their cuts along K.
 constexpr int kShortTileRows = 64;
 constexpr size_t kCutSlotBytes = (size_t)8 * kTN * 256 * 4;  // a work item's partial sums: 8 wavefronts x 16 x 128 floats
+constexpr int kTableMinGroups = 24;
+size_t tile_table_bytes(int64_t tile_rows) { return (size_t)(tile_rows + 1) * sizeof(int4); }
 // Largest number of cuts per tile of the last round, as a shift (the kernel picks among 0..this from the real tile
 // count): whole K-blocks, at least 8 per cut, and slots for a round short of one tile.
 // (256-row tiles, jn = 4: a round short of one tile would need four times the slots; the kernel, which knows how many
@@ -1460,6 +1527,16 @@ int launch_block(const GemmArgs& g, int mode, void* workspace, size_t workspace_
     FG_CHECK_LAUNCH("transpose_scales_kernel");
     a.g.xs = xs_t; a.g.xs_rs = 1; a.g.xs_cs = scale_rows;
   }
+  if (grouped != nullptr && a.n_groups >= kTableMinGroups && a.n_groups <= kTableGroups && workspace != nullptr) {
+    const size_t at = need + transposed_scales_bytes(scale_rows, g.KB);
+    if ((uintptr_t)workspace % 16 == 0 && workspace_bytes >= at + tile_table_bytes(a.g.tiles_m)) {
+      int4* const table = reinterpret_cast<int4*>(reinterpret_cast<uint8_t*>(workspace) + at);
+      FG_LAUNCH(group_tile_rows_kernel, dim3(1), dim3(1024), 0, stream, a.groups, a.n_groups, g.M,
+                short_tiles ? kShortTileRows * short_jn : kBM, a.g.tiles_m, table);
+      FG_CHECK_LAUNCH("group_tile_rows_kernel");
+      a.tile_rows = table;
+    }
+  }
   if (sk.use && mode < kModeRowColBF16 && workspace != nullptr && workspace_bytes >= need && (size_t)sk.grid * 8 * 4 <= FG_WORKSPACE_COUNTER_BYTES &&
       (uintptr_t)workspace % 16 == 0) {
     a.sk = 1; a.sk_q = sk.q; a.sk_r = sk.r; a.sk_split = sk.split;
@@ -1549,7 +1626,8 @@ size_t pingpong_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 size_t grouped_workspace_bytes(int64_t M, int64_t K) {
   if (M <= 0 || K <= 0 || K % 128 != 0) return 0;
   // (the partial sums of cut short tiles: the number of segments is not known here, the bound of the plan is)
-  return FG_WORKSPACE_COUNTER_BYTES + (size_t)kMaxCutItems * kCutSlotBytes + transposed_scales_bytes(M, K / 128);
+  return FG_WORKSPACE_COUNTER_BYTES + (size_t)kMaxCutItems * kCutSlotBytes + transposed_scales_bytes(M, K / 128) +
+         tile_table_bytes(M);  // (a tile row holds at least one row)
 }
 
 int launch_grouped(const GemmArgs& g, const GroupedGemm& grouped, void* workspace, size_t workspace_bytes, hipStream_t stream) {
