@@ -1,5 +1,5 @@
-// Device code shared by the tile kernels whose wavefront groups alternate between fetching and multiplying
-// (fp8_gemm_pingpong.hip, fp8_gemm_alternating.hip): fragments in LDS, matrix instructions written out in assembly, and
+// Device code of the persistent kernel, whose wavefront groups alternate between fetching and multiplying
+// (fp8_gemm_pingpong.hip): fragments in LDS, matrix instructions written out in assembly, and
 // the stores of a wavefront's results.
 #pragma once
 

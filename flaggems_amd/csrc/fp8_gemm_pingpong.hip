@@ -463,7 +463,8 @@ __device__ __forceinline__ void finish_cut_tile(const PpArgs& a, const v4f (&acc
 // 64th are loaded like rows past an edge and never read), and everything else runs unchanged.
 // F16: the results are fp16 (else bf16).  A template parameter and not a test of c_dtype in the flush: with both
 // forms of the stores in one kernel the bf16 flush of short-K problems got 5 % slower.
-template <bool SK, int MODE, bool ALIGNED, bool GROUPED = false, bool POW2 = false, int JN = kTM, bool F16 = false>
+// GATHER (grouped problems): the activation rows may be read through a.gather_index.
+template <bool SK, int MODE, bool ALIGNED, bool GROUPED = false, bool POW2 = false, int JN = kTM, bool F16 = false, bool GATHER = GROUPED>
 __global__ __launch_bounds__(kThreads) void fp8_gemm_pingpong_kernel(PpArgs a) {
   static_assert(JN == kTM || (GROUPED && JN >= 1 && JN < kTM), "short tiles: grouped problems only");
   constexpr int kTileRows = 64 * JN;
@@ -560,7 +561,7 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_pingpong_kernel(PpArgs a) {
   lw.start(a, first_idx, first_kb, n_tiles, tiles_m);
   LoadShare share = {};
   auto set_load_tile = [&]() __attribute__((always_inline)) {
-    if (GROUPED && a.gather_index != nullptr && wave < 4) {
+    if (GATHER && a.gather_index != nullptr && wave < 4) {
       const int valid = lw.m_end - lw.m0;
       share.set_gathered(g, a.gather_index, a.index_div, a.x_rows, lw.m0, valid < kTileRows ? valid : kTileRows, lane, wave);
     } else {
@@ -605,7 +606,7 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_pingpong_kernel(PpArgs a) {
   uint32_t xs_off[kTM] = {0u, 0u, 0u, 0u};
   const float* xs_ptr = g.xs;
   // offsets are relative to the tile's first row; rows past the edge read the last row's scale
-  const bool gathered = GROUPED && a.gather_index != nullptr;  // uniform
+  const bool gathered = GATHER && a.gather_index != nullptr;  // uniform
   auto set_scale_offsets = [&]() __attribute__((always_inline)) {
 #pragma unroll
     for (int j = 0; j < kTM; ++j) {
@@ -1019,6 +1020,41 @@ bool transposition_pays(int64_t tiles, int64_t KB, int cus) {
 }
 size_t transposed_scales_bytes(int64_t M, int64_t KB) { return (size_t)((M * KB * 4 + 255) / 256 * 256); }
 
+// Activation rows of a grouped problem in sorted order (row m = row row_index[m] / index_div of X, forced into
+// [0, x_rows)), and their scales, transposed as above.  A block takes 16 consecutive rows.
+constexpr int kGatherRows = 16;
+__global__ __launch_bounds__(256) void gather_rows_kernel(const uint8_t* __restrict__ X, int64_t ldx, const float* __restrict__ xs, int64_t rs, int64_t cs,
+                                                          const int* __restrict__ row_index, int index_div, int x_rows, int M, int K,
+                                                          uint8_t* __restrict__ out, float* __restrict__ out_scales) {
+  __shared__ int s_src[kGatherRows];
+  const int m0 = (int)blockIdx.x * kGatherRows, tid = (int)threadIdx.x;
+  const int rows = M - m0 < kGatherRows ? M - m0 : kGatherRows;
+  if (tid < rows) {
+    const int src = row_index[m0 + tid] / index_div;
+    s_src[tid] = src < 0 ? 0 : (src < x_rows ? src : x_rows - 1);
+  }
+  __syncthreads();
+  const int chunks = K >> 4;  // 16 bytes each (K is a multiple of 128)
+  for (int r = tid >> 6; r < rows; r += 4) {
+    const u32x4* const from = reinterpret_cast<const u32x4*>(X + (int64_t)s_src[r] * ldx);
+    u32x4* const to = reinterpret_cast<u32x4*>(out + (int64_t)(m0 + r) * K);
+#pragma unroll 4
+    for (int c = tid & 63; c < chunks; c += 64) to[c] = from[c];
+  }
+  const int r = tid & (kGatherRows - 1);
+  if (r < rows)
+    for (int kb = tid / kGatherRows; kb < (K >> 7); kb += 256 / kGatherRows)
+      out_scales[(int64_t)kb * M + m0 + r] = xs[(int64_t)s_src[r] * rs + (int64_t)kb * cs];
+}
+// Where it pays.  Reading 256-row tiles through the index costs a block about 10 us at every tile: index loads and their
+// divisions, whose waits cover every copy in flight, in two walks.  The copy moves 2 M K bytes once and is a launch (4096
+// tokens twice, K = 4096: 12 us); 8192 rows, 8 segments, [28672, 4096], 15.8 tiles a block: GEMM 1212 -> 1041 us.
+constexpr size_t kMaxGatheredBytes = (size_t)1 << 30;
+size_t gathered_bytes(int64_t M, int64_t K) { return (size_t)((M * K + 255) / 256 * 256); }
+bool gather_copy_pays(int64_t M, int64_t K, int64_t tiles, int cus) {
+  return gathered_bytes(M, K) <= kMaxGatheredBytes && (double)tiles / cus * 6.0 > 5.0 + (double)M * (double)K * 2 / 5e6;
+}
+
 // Tile rows of a grouped problem (PpArgs::tile_rows).  One block: the group ends, forced into ascending order and into
 // [0, M] as segment_end does, and the tile rows before every group by scans in LDS; then every tile row finds its group
 // by bisection.  Latency-bound, about 4 us; it pays from a few dozen groups on, because a walk that scans the table
@@ -1076,7 +1112,9 @@ __global__ __launch_bounds__(1024) void group_tile_rows_kernel(const int* ends, 
 // Short tiles of grouped problems (the JN = 1 instantiation) and their cuts along K.
 constexpr int kShortTileRows = 64;
 constexpr size_t kCutSlotBytes = (size_t)8 * kTN * 256 * 4;  // a work item's partial sums: 8 wavefronts x 16 x 128 floats
-constexpr int kTableMinGroups = 24;
+// A launch of one block, about 5 us, against a scan of about 0.1 us a group in each of three walks at every tile a block
+// enters: from some two dozen (groups x tiles a block) on.  8 groups, 15.8 tiles a block (8192 rows, [28672, 4096]): 1243 -> 1212 us.
+constexpr int64_t kTableMinScans = 24;
 size_t tile_table_bytes(int64_t tile_rows) { return (size_t)(tile_rows + 1) * sizeof(int4); }
 // Largest number of cuts per tile of the last round, as a shift (the kernel picks among 0..this from the real tile
 // count): whole K-blocks, at least 8 per cut, and slots for a round short of one tile.
@@ -1094,13 +1132,15 @@ struct KernelChoice {
   int short_jn;  // grouped problems on short tiles: 16-row fragments per wavefront (1 or 2), else 0
   int mode;
   bool sk, aligned, pow2;
+  bool gather;   // grouped problems on 256-row tiles: rows read through an index in the kernel
 };
 template <bool F16>
 void (*pick_kernel(const KernelChoice& c))(PpArgs) {
   if (c.grouped)
     return c.short_jn == 1   ? fp8_gemm_pingpong_kernel<false, kModeBlock, false, true, false, 1, F16>
            : c.short_jn == 2 ? fp8_gemm_pingpong_kernel<false, kModeBlock, false, true, false, 2, F16>
-                             : fp8_gemm_pingpong_kernel<false, kModeBlock, false, true, false, kTM, F16>;
+           : c.gather        ? fp8_gemm_pingpong_kernel<false, kModeBlock, false, true, false, kTM, F16, true>
+                             : fp8_gemm_pingpong_kernel<false, kModeBlock, false, true, false, kTM, F16, false>;
   if (c.mode == kModeRowColI8) {
     if (c.sk)
       return c.aligned ? fp8_gemm_pingpong_kernel<true, kModeRowColI8, true, false, false, kTM, F16>
@@ -1227,7 +1267,20 @@ int launch_block(const GemmArgs& g, int mode, void* workspace, size_t workspace_
   // workspace: [counters][partial tiles, if the shape is one that shares tiles][transposed activation scales]
   // (a grouped problem's tile count is an upper bound that a few hundred rows spread over many segments inflate:
   // there the gathers are few and the transposition, ~5 us whatever the size, does not pay)
-  if (mode == kModeBlock && g.xs_rs >= kTransposeMinRowStride && transposition_pays(tiles, g.KB, cus) && workspace != nullptr &&
+  size_t at = need + transposed_scales_bytes(scale_rows > g.M ? scale_rows : g.M, g.KB);  // what follows the scales
+  if (a.gather_index != nullptr && !short_tiles && workspace != nullptr && (uintptr_t)workspace % 16 == 0 && g.K % 128 == 0 &&
+      g.ldx % 16 == 0 && (uintptr_t)g.X % 16 == 0 && gather_copy_pays(g.M, g.K, tiles, cus) &&
+      workspace_bytes >= at + gathered_bytes(g.M, g.K)) {
+    float* const xs_t = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + need);
+    uint8_t* const rows = reinterpret_cast<uint8_t*>(workspace) + at;
+    FG_LAUNCH(gather_rows_kernel, dim3((uint32_t)ceil_div(g.M, kGatherRows)), dim3(256), 0, stream, g.X, g.ldx, g.xs, g.xs_rs, g.xs_cs, a.row_index,
+              a.index_div, a.x_rows, g.M, g.K, rows, xs_t);
+    FG_CHECK_LAUNCH("gather_rows_kernel");
+    a.g.X = rows; a.g.ldx = g.K;
+    a.g.xs = xs_t; a.g.xs_rs = 1; a.g.xs_cs = g.M;
+    a.gather_index = nullptr;
+    at += gathered_bytes(g.M, g.K);
+  } else if (mode == kModeBlock && g.xs_rs >= kTransposeMinRowStride && transposition_pays(tiles, g.KB, cus) && workspace != nullptr &&
       (grouped == nullptr || g.M >= 1024) &&
       (uintptr_t)workspace % 16 == 0 &&
       workspace_bytes >= need + transposed_scales_bytes(scale_rows, g.KB)) {
@@ -1237,8 +1290,7 @@ int launch_block(const GemmArgs& g, int mode, void* workspace, size_t workspace_
     FG_CHECK_LAUNCH("transpose_scales_kernel");
     a.g.xs = xs_t; a.g.xs_rs = 1; a.g.xs_cs = scale_rows;
   }
-  if (grouped != nullptr && a.n_groups >= kTableMinGroups && a.n_groups <= kTableGroups && workspace != nullptr) {
-    const size_t at = need + transposed_scales_bytes(scale_rows, g.KB);
+  if (grouped != nullptr && a.n_groups * (tiles > cus ? tiles / cus : 1) >= kTableMinScans && a.n_groups <= kTableGroups && workspace != nullptr) {
     if ((uintptr_t)workspace % 16 == 0 && workspace_bytes >= at + tile_table_bytes(a.g.tiles_m)) {
       int4* const table = reinterpret_cast<int4*>(reinterpret_cast<uint8_t*>(workspace) + at);
       FG_LAUNCH(group_tile_rows_kernel, dim3(1), dim3(1024), 0, stream, a.groups, a.n_groups, g.M,
@@ -1265,7 +1317,7 @@ int launch_block(const GemmArgs& g, int mode, void* workspace, size_t workspace_
   const bool aligned = g.M % kBM == 0 && g.N % kBN == 0;
   const bool pow2 = mode == kModeBlock && grouped == nullptr && g.scales_pow2 != 0;
   const bool f16 = g.c_dtype == FG_F16;
-  const KernelChoice which = {grouped != nullptr, short_jn, mode, a.sk != 0, aligned, pow2};
+  const KernelChoice which = {grouped != nullptr, short_jn, mode, a.sk != 0, aligned, pow2, a.gather_index != nullptr};
   void (*const kern)(PpArgs) = f16 ? pick_kernel<true>(which) : pick_kernel<false>(which);
   if (const int rc = allow_full_lds(kern)) return rc;
   if (tp.use && !a.sk && workspace != nullptr && workspace_bytes >= need && (size_t)tp.grid * 8 * 4 <= FG_WORKSPACE_COUNTER_BYTES &&
@@ -1337,7 +1389,8 @@ size_t grouped_workspace_bytes(int64_t M, int64_t K) {
   if (M <= 0 || K <= 0 || K % 128 != 0) return 0;
   // (the partial sums of cut short tiles: the number of segments is not known here, the bound of the plan is)
   return FG_WORKSPACE_COUNTER_BYTES + (size_t)kMaxCutItems * kCutSlotBytes + transposed_scales_bytes(M, K / 128) +
-         tile_table_bytes(M);  // (a tile row holds at least one row)
+         tile_table_bytes(M) +  // (a tile row holds at least one row)
+         (M >= 1024 && gathered_bytes(M, K) <= kMaxGatheredBytes ? gathered_bytes(M, K) : 0);
 }
 
 int launch_grouped(const GemmArgs& g, const GroupedGemm& grouped, void* workspace, size_t workspace_bytes, hipStream_t stream) {
