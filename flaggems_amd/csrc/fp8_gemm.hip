@@ -677,6 +677,7 @@ int launch_tile_split(GemmArgs a, const TileSplitPlan& plan, void* workspace, hi
 // second round of this kernel loses to the persistent kernel (M = 1024, N = 4608, K = 7168, 288 tiles: 62 -> 79 us).
 struct PipePlan {
   bool use;
+  bool tall;  // 256 x 128 tiles, three stages
   int splits, kb_per_split;
   size_t workspace_bytes;
 };
@@ -693,13 +694,27 @@ bool mid_m_partial_round(const MidMPlan& mid, int cus) {
 }
 
 PipePlan plan_pipe(int64_t M, int64_t N, int64_t K, int64_t xs_rs, int64_t entries = 1) {
-  PipePlan p = {false, 1, 0, 0};
+  PipePlan p = {false, false, 1, 0, 0};
   if (entries < 1) entries = 1;
   if (M <= 16 || (M <= 32 && entries > 1) || K <= 0 || K % 128 != 0) return p;
   if (xs_rs < 0 || xs_rs >= (1 << 21)) return p;  // 256 rows of scales addressed with 32-bit byte offsets
   const int64_t KB = K / 128;
   const int64_t tiles = ceil_div(M, kSplitTile) * ceil_div(N, kSplitTile) * entries;
   const int cus = cu_count();
+  // More 128-row tiles than compute units, but no more 256-row ones (so over half of the units get one): 256 x 128 tiles in
+  // one round.  Two rounds of 128-row tiles, or the persistent kernel's 256 x 256 tiles, cut along K and put together through
+  // the workspace, are the alternatives; us: M = 300, N = 14336, K = 4096: 47.8 -> 41.3; M = 2048, N = K = 4096: 47.1 -> 42.0; M = 1000,
+  // N = 7168, K = 2304: 28.4 -> 26.3; M = 3000, N = 2112, K = 7168: 69.7 -> 62.5; row and column scales: M = 500, N = 10240, K = 8192: 92.8 ->
+  // 70.5, M = 2000, N = 4096, K = 7168: 75.6 -> 59.5.  Not with four K-blocks (M = 256, N = 20480, K = 512: 11.9 -> 12.3), nor with
+  // long K on few units (M = 1000, N = 4608, K = 7168, 144 tiles: 58.5 -> 59.9), which the persistent kernel's cuts fill.  Split along K
+  // such tiles lose to 128-row ones (M = 256: N = K = 8192 in four: 36.5 -> 41.4): twice the partial sums.
+  if (entries == 1 && M > 128 && tiles > cus && KB >= 8 && KB <= 64) {
+    const int64_t tall = ceil_div(M, (int64_t)2 * kSplitTile) * ceil_div(N, kSplitTile);
+    if (tall > cus || (KB > 32 && tall * 10 < (int64_t)cus * 6)) return p;
+    p.tall = p.use = true;
+    p.kb_per_split = (int)KB;
+    return p;
+  }
   if (tiles > cus || KB < 4) return p;
   if (tiles * kSplitWaves * 4 > FG_WORKSPACE_COUNTER_BYTES) return p;
   int64_t splits = cus / tiles;
@@ -748,17 +763,17 @@ PipePlan plan_pipe(int64_t M, int64_t N, int64_t K, int64_t xs_rs, int64_t entri
   return p;
 }
 
-template <int MODE>
-int launch_pipe(GemmArgs a, const PipePlan& plan, void* workspace, hipStream_t stream) {
-  using Cfg = TileCfg<kSplitTile, kSplitTile, kSplitWM, 2, kPipeStages>;
-  a.tiles_m = (int)ceil_div(a.M, kSplitTile);
+template <int MODE, int BM, int NST>
+int launch_pipe_tile(GemmArgs a, const PipePlan& plan, void* workspace, hipStream_t stream) {
+  using Cfg = TileCfg<BM, kSplitTile, kSplitWM, 2, NST>;
+  a.tiles_m = (int)ceil_div(a.M, BM);
   a.tiles_n = (int)ceil_div(a.N, kSplitTile);
   a.splits = plan.splits;
   a.kb_per_split = plan.kb_per_split;
   a.split_counters = reinterpret_cast<unsigned int*>(workspace);
   a.split_partials = workspace && plan.splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + FG_WORKSPACE_COUNTER_BYTES) : nullptr;
-  a.split_partials_per_entry = (int64_t)a.tiles_m * a.tiles_n * a.splits * kSplitTile * kSplitTile;
-  auto kern = fp8_gemm_kernel<kSplitTile, kSplitTile, kSplitWM, 2, MODE, true, true, kPipeStages>;
+  a.split_partials_per_entry = (int64_t)a.tiles_m * a.tiles_n * a.splits * BM * kSplitTile;
+  auto kern = fp8_gemm_kernel<BM, kSplitTile, kSplitWM, 2, MODE, true, true, NST>;
   static PerDeviceFlags lds_limit_raised = {};
   {
     const hipError_t e = raise_dynamic_lds_limit(lds_limit_raised, Cfg::kLdsBytes, reinterpret_cast<const void*>(kern));
@@ -766,8 +781,14 @@ int launch_pipe(GemmArgs a, const PipePlan& plan, void* workspace, hipStream_t s
   }
   const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n * a.splits;
   FG_LAUNCH(kern, dim3((uint32_t)blocks, (uint32_t)(a.batch > 1 ? a.batch : 1)), dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, a);
-  FG_CHECK_LAUNCH("fp8_gemm_kernel (four stages)");
+  FG_CHECK_LAUNCH("fp8_gemm_kernel (deep pipeline)");
   return FG_OK;
+}
+
+template <int MODE>
+int launch_pipe(const GemmArgs& a, const PipePlan& plan, void* workspace, hipStream_t stream) {
+  if (plan.tall) return launch_pipe_tile<MODE, 2 * kSplitTile, 3>(a, plan, workspace, stream);
+  return launch_pipe_tile<MODE, kSplitTile, kPipeStages>(a, plan, workspace, stream);
 }
 
 // Parts of up to 16 rows in which the decode kernels take 17..512 rows of a lone problem (measurements at the call): two, four,
