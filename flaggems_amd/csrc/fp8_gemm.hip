@@ -166,6 +166,7 @@ __device__ __forceinline__ void scale_accumulate(v4f& acc, const v4f& p, float s
 // Global -> LDS copies the compiler does not see (it would otherwise order every later LDS read behind them):
 // 16 bytes per lane to lds_addr + 16 * lane, or 4 bytes per lane to lds_addr + 4 * lane.  `base` and `lds_addr`
 // are wave-uniform; the copy counts in vmcnt and has landed in LDS when the counter says so.
+// (Distance between a base that a vector instruction wrote and the copy: see store_x4_agent.)
 __device__ __forceinline__ void copy_to_lds_16(uint32_t byte_off, const void* base, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\t"
                "s_nop 0\n\t"

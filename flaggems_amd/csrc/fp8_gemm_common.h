@@ -202,7 +202,9 @@ __device__ __forceinline__ T* uniform_ptr(T* p) {
 // compiler's wait-count insertion: callers wait explicitly.  The base may have come out of v_readfirstlane or v_readlane
 // (a spilled scalar) in the instruction before: a vector-memory instruction must not read a scalar register within five
 // wait states of a vector instruction that wrote it, and the compiler keeps that distance only for instructions of its
-// own, hence the s_nop.
+// own, hence the s_nop.  (The global -> LDS copies of the GEMM kernels have scalar bases too; there three more wait states a
+// copy, or a scalar copy of the base, cost up to 3 %: M = 1000, N = 2112, K = 7168: 38.8 -> 40.3 and 39.7 us.  They go
+// without: tests/test_scalar_base_distance.py looks through the machine code of every build for a base read too early.)
 __device__ __forceinline__ void store_x4_agent(float* base, uint32_t byte_off, const v4f& v) {
   asm volatile("s_nop 4\n\tglobal_store_dwordx4 %0, %1, %2 sc1" : : "v"(byte_off), "v"(v), "s"(base) : "memory");
 }

@@ -287,7 +287,8 @@ struct LoadShare {
   // The load is written out instead of using the compiler's builtin: the compiler books a global->LDS
   // load as an access that may return through either counter, and from then on turns every wait for an LDS
   // read into lgkmcnt(0), which makes the multiply phase wait for fragments it needs two rows later.
-  // stage_lds: LDS byte address of this wavefront's first slab in the stage (uniform).
+  // stage_lds: LDS byte address of this wavefront's first slab in the stage (uniform).  (Distance between a base that a vector
+  // instruction wrote and the load, here and in load_f32_untracked: see store_x4_agent.)
   __device__ __forceinline__ void issue_one(uint32_t stage_lds, int q) const {
     asm volatile("s_add_u32 m0, %2, %3\n\t"
                  "s_nop 0\n\t"

@@ -280,6 +280,7 @@ struct PairRegs {
 
 // Global -> LDS copies the compiler does not see: 16 (4) bytes per lane to lds_addr + 16 (4) * lane.  `base` and
 // `lds_addr` are wave-uniform; the copies count in vmcnt like loads and complete in order with them.
+// (Distance between a base that a vector instruction wrote and the copy: see store_x4_agent.)
 __device__ __forceinline__ void dma_to_lds_16(uint32_t byte_off, const void* base, uint32_t lds_addr) {
   asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(byte_off), "s"(base), "s"(lds_addr) : "memory", "m0");
 }
