@@ -17,6 +17,7 @@
 // MFMA accumulates directly and the scales are applied once in the epilogue.
 
 #include "fp8_gemm_common.h"
+#include "fp8_gemm_rules.h"
 
 #include <mutex>
 #include <type_traits>
@@ -694,7 +695,7 @@ bool mid_m_partial_round(const MidMPlan& mid, int cus) {
   return rounds >= 2 && blocks * 10 < rounds * slots * 9;
 }
 
-PipePlan plan_pipe(int64_t M, int64_t N, int64_t K, int64_t xs_rs, int64_t entries = 1) {
+PipePlan plan_pipe(bool block_scales, int64_t M, int64_t N, int64_t K, int64_t xs_rs, int64_t entries = 1) {
   PipePlan p = {false, false, 1, 0, 0};
   if (entries < 1) entries = 1;
   if (M <= 16 || (M <= 32 && entries > 1) || K <= 0 || K % 128 != 0) return p;
@@ -702,16 +703,7 @@ PipePlan plan_pipe(int64_t M, int64_t N, int64_t K, int64_t xs_rs, int64_t entri
   const int64_t KB = K / 128;
   const int64_t tiles = ceil_div(M, kSplitTile) * ceil_div(N, kSplitTile) * entries;
   const int cus = cu_count();
-  // More 128-row tiles than compute units, but no more 256-row ones (so over half of the units get one): 256 x 128 tiles in
-  // one round.  Two rounds of 128-row tiles, or the persistent kernel's 256 x 256 tiles, cut along K and put together through
-  // the workspace, are the alternatives; us: M = 300, N = 14336, K = 4096: 47.8 -> 41.3; M = 2048, N = K = 4096: 47.1 -> 42.0; M = 1000,
-  // N = 7168, K = 2304: 28.4 -> 26.3; M = 3000, N = 2112, K = 7168: 69.7 -> 62.5; row and column scales: M = 500, N = 10240, K = 8192: 92.8 ->
-  // 70.5, M = 2000, N = 4096, K = 7168: 75.6 -> 59.5.  Not with four K-blocks (M = 256, N = 20480, K = 512: 11.9 -> 12.3), nor with
-  // long K on few units (M = 1000, N = 4608, K = 7168, 144 tiles: 58.5 -> 59.9), which the persistent kernel's cuts fill.  Split along K
-  // such tiles lose to 128-row ones (M = 256: N = K = 8192 in four: 36.5 -> 41.4): twice the partial sums.
-  if (entries == 1 && M > 128 && tiles > cus && KB >= 8 && KB <= 64) {
-    const int64_t tall = ceil_div(M, (int64_t)2 * kSplitTile) * ceil_div(N, kSplitTile);
-    if (tall > cus || (KB > 32 && tall * 10 < (int64_t)cus * 6)) return p;
+  if (entries == 1 && tall_tiles_pay(block_scales, M, N, KB, cus)) {
     p.tall = p.use = true;
     p.kb_per_split = (int)KB;
     return p;
@@ -936,7 +928,7 @@ int launch_gemm(const GemmArgs& a, void* workspace, size_t workspace_bytes, hipS
       if (sp.use && sp.own) return launch_small_m(a, MODE, sp, workspace, workspace_bytes, stream);
     }
     if (a.M <= 64) {  // the four-stage tile kernel where its planner prefers it to the staged-activation and decode kernels
-      const PipePlan pp = plan_pipe(a.M, a.N, a.K, MODE == kModeBlock ? a.xs_rs : 0);
+      const PipePlan pp = plan_pipe(MODE == kModeBlock, a.M, a.N, a.K, MODE == kModeBlock ? a.xs_rs : 0);
       const bool ws_ok = pp.splits == 1 || (workspace != nullptr && workspace_bytes >= pp.workspace_bytes && (uintptr_t)workspace % 16 == 0);
       if (pp.use && ws_ok) return launch_pipe<MODE>(a, pp, workspace, stream);
     }
@@ -944,7 +936,7 @@ int launch_gemm(const GemmArgs& a, void* workspace, size_t workspace_bytes, hipS
                                           (uintptr_t)workspace % 16 == 0)))
       return launch_mid_m(a, MODE, mid, workspace, workspace_bytes, stream);
     {
-      const PipePlan pp = plan_pipe(a.M, a.N, a.K, MODE == kModeBlock ? a.xs_rs : 0);
+      const PipePlan pp = plan_pipe(MODE == kModeBlock, a.M, a.N, a.K, MODE == kModeBlock ? a.xs_rs : 0);
       const bool ws_ok = pp.splits == 1 || (workspace != nullptr && workspace_bytes >= pp.workspace_bytes && (uintptr_t)workspace % 16 == 0);
       if (pp.use && ws_ok && !mid_takes) return launch_pipe<MODE>(a, pp, workspace, stream);
     }
@@ -1006,7 +998,7 @@ int check_common(const void* A, const void* B, const void* C, int64_t lda, int64
 extern "C" size_t fg_block_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K) {
   // the largest any kernel that may take the shape can use
   size_t need = fg::plan_tile_split(M, N, K).workspace_bytes;
-  const fg::PipePlan pipe = fg::plan_pipe(M, N, K, 0);
+  const fg::PipePlan pipe = fg::plan_pipe(true, M, N, K, 0);
   if (pipe.use && pipe.workspace_bytes > need) need = pipe.workspace_bytes;
   const fg::SmallMPlan plan = fg::plan_small_m(M, N, K);
   if (plan.use && plan.workspace_bytes > need) need = plan.workspace_bytes;
@@ -1169,7 +1161,7 @@ extern "C" size_t fg_batched_block_fp8_gemm_workspace_bytes(int64_t batch, int64
     }
   }
   if (batch > 1) {
-    const fg::PipePlan pipe = fg::plan_pipe(M, N, K, 0, batch);
+    const fg::PipePlan pipe = fg::plan_pipe(true, M, N, K, 0, batch);
     if (pipe.use && pipe.workspace_bytes > need) need = pipe.workspace_bytes;
   }
   return need;
@@ -1223,7 +1215,7 @@ extern "C" int fg_batched_block_fp8_gemm(const void* A, int64_t lda, int64_t a_b
       }
       {
         // few tiles in the whole batch: the four-stage tile kernel, K split over blocks until the compute units are full
-        const PipePlan pp = plan_pipe(M, N, K, as_row_stride, batch);
+        const PipePlan pp = plan_pipe(true, M, N, K, as_row_stride, batch);
         const bool fits = pp.splits == 1 || (workspace != nullptr && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= pp.workspace_bytes);
         if (pp.use && fits) return launch_pipe<kModeBlock>(a, pp, workspace, (hipStream_t)stream);
       }
