@@ -35,4 +35,34 @@ inline bool tall_tiles_pay(bool block_scales, int64_t M, int64_t N, int64_t k_bl
   return M <= 256 ? k_blocks > (many ? 16 : 20) : M <= 512 && k_blocks > 24 && many;
 }
 
+// Few rows a group: activation rows a pass of the weight-streaming grouped kernel takes (16, 32 or 64), or 0 where the persistent
+// kernel's 64- to 256-row tiles are faster.  The host knows the rows of an average group only; longer groups take several passes,
+// which find their weights in a cache.  us, streaming / persistent, groups x [N, K], rows a group:
+//   8 x [28672, 4096]: 6: 166 / 202   16: 178 / 198   32: 187 / 219   48: 198 / 238   64: 263 / 238
+//   8 x [4096, 14336]: 6:  84 / 112   16:  84 / 113   32:  89 / 111   48:  96 / 117   64: 137 / 120
+//   64 x [2048, 4096]: 48: 135 / 142  64: 177 / 144
+//   512 x [2048, 4096]: 1: 468 / 2348 (before its table of tile rows)   16: 804 / -   32: 912 / 816   48: 1009 / 869
+// With few groups the persistent kernel loses its last round of tiles, with many it does not.  Hence the 24 rows (48 up to 64
+// groups), and
+//   * large matrices in 32 groups or more: only up to 32 rows, past which its 128-row tiles stop at one a group.  32 x [4096, 14336]:
+//     30: 357 / 393   34: 368 / 336   48: 386 / 339; unequal groups (shares falling as the root of the rank) 30: 404 / 440   48: 471 / 402.
+//     (26 x [4096, 14336], unequal: 37: 333 / 404; 64 x [2816, 2048]: 48: 92 / 98.)
+//   * one or two K-blocks and no more 256-wide tiles than compute units: an item is a single step, and the table of groups in front
+//     and the exchange behind it cost 2 - 5 us more than they save, up to about a dozen groups, whose table the persistent kernel
+//     scans as quickly.  K = 256: 2 x 7168: 1: 12.8 / 10.7   40: 16.8 / 12.2; 8 x 2048: 1: 12 / 11.  (K = 384: 2 x 7168: 1: 11 / 13;
+//     K = 256, 16 x 2048: 1: 13 / 16; 8 x 16384, two rounds: 1: 13 / 20.)
+// A pass of 16 rows streams fastest (4 stages in flight), 32 are 1 - 3 % slower; 64 another 3 - 9 %.  Where one group holds every row
+// the passes repeat: 8 x [28672, 4096], 64 rows, 16 a pass 71, 32 a pass 41, persistent 41.  So large matrices, whose passes cost
+// most and where the wider pass costs least (8 x [4096, 14336], 64 rows: 84.6 and 84.8 spread evenly, 93 and 88 with unequal groups),
+// take 32 rows from 4 a group on (from 17 rows in all: 1 x [4096, 6400], 5 rows: 15.1 with 16 a pass, 16.7 with 32).  With everything in one group the kernel stays up to 1.8 times slower than the persistent one on large
+// matrices (64 x [4096, 14336], 1024 rows: 254 / 144); spread as routers spread them it is faster.
+inline int grouped_stream_pass_rows(int64_t M, int64_t N, int64_t k_blocks, int64_t groups, int64_t cus) {
+  const bool large = N * k_blocks * 128 >= 24000000;
+  if (k_blocks <= 2 && groups * ((N + 255) / 256) <= cus && groups <= (k_blocks == 1 || M > 24 * groups ? 12 : 8)) return 0;
+  if (M <= 16 || M <= (large ? 4 : 8) * groups) return 16;
+  if (M <= 24 * groups) return 32;
+  if (M <= 32 * groups) return groups <= 64 ? 64 : 0;
+  return M <= 48 * groups && groups <= (large ? 31 : 64) ? 64 : 0;
+}
+
 }  // namespace fg

@@ -31,6 +31,7 @@
 // wavefront reads together fall into 16 different bank groups.
 
 #include "fp8_gemm_common.h"
+#include "fp8_gemm_rules.h"
 
 namespace fg {
 namespace {
@@ -494,17 +495,7 @@ int grouped_stream_rows(const GemmArgs& g, const GroupedGemm& gr) {
   // steps are counted in 32 bits
   const int64_t chunks = ceil_div(g.N, (int64_t)kItemCols), pairs = (g.KB + 1) / 2;
   if ((g.M / 16 + E) * chunks * pairs >= (1ll << 30)) return 0;
-  // Rows a pass by the average group (the host knows no more; longer groups take several passes, and the second finds
-  // its weights in the memory-side cache).  Past these the persistent kernel's 64- and 128-row tiles are faster: with few
-  // groups it loses its last round of tiles, with many it does not.  us, this kernel / the persistent kernel, by rows a
-  // group, groups x [N, K]:
-  //   8 x [28672, 4096]: 6: 166 / 202   16: 178 / 198   32: 187 / 219   48: 198 / 238   64: 263 / 238
-  //   8 x [4096, 14336]: 6:  84 / 112   16:  84 / 113   32:  89 / 111   48:  96 / 117   64: 137 / 120
-  //   64 x [2048, 4096]: 48: 135 / 142  64: 177 / 144
-  //   512 x [2048, 4096]: 1: 468 / 2348 (before its table of tile rows)   16: 804 / -   32: 912 / 816   48: 1009 / 869
-  if (g.M <= 8 * E) return 16;
-  if (g.M <= 24 * E) return 32;
-  return E <= 64 && g.M <= 48 * E ? 64 : 0;
+  return grouped_stream_pass_rows(g.M, g.N, g.KB, E, cu_count());
 }
 
 size_t stream_workspace_bytes() { return FG_WORKSPACE_COUNTER_BYTES + (size_t)512 * part_bytes(4); }

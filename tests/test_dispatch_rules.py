@@ -11,6 +11,9 @@ HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))
 SHIM = """
 #include "%s"
 extern "C" int tall(int block, long long M, long long N, long long kb, long long cus) { return fg::tall_tiles_pay(block != 0, M, N, kb, cus); }
+extern "C" int stream_rows(long long M, long long N, long long kb, long long groups, long long cus) {
+  return fg::grouped_stream_pass_rows(M, N, kb, groups, cus);
+}
 """ % HEADER
 
 
@@ -26,6 +29,7 @@ def rules(tmp_path_factory):
     subprocess.run([cxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-o", lib, src], check=True)
     so = ctypes.CDLL(lib)
     so.tall.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
+    so.stream_rows.argtypes = [ctypes.c_longlong] * 5
     return so
 
 
@@ -58,3 +62,31 @@ def test_tall_tiles_only_where_one_round_takes_them(rules, block):
                     if rules.tall(block, M, N, kb, cus):
                         assert M > 128 and 8 <= kb <= 64
                         assert -(-M // 256) * -(-N // 128) <= cus < -(-M // 128) * -(-N // 128)
+
+
+# groups, N, K, rows a group, us on the streaming kernel, us on the persistent one (rows spread at random over the groups)
+STREAM = [
+    (1, 7168, 256, 4, 12.3, 10.0), (2, 7168, 256, 1, 12.8, 10.7), (2, 2048, 256, 48, 16.3, 11.8), (4, 7168, 128, 32, 15.3, 11.4),
+    (8, 7168, 128, 48, 17.0, 13.4), (8, 7168, 256, 48, 17.7, 14.9),
+    (8, 16384, 256, 1, 13.0, 20.1), (16, 7168, 256, 24, 15.0, 21.6), (16, 2048, 256, 1, 13.0, 16.0), (256, 7168, 256, 12, 119.6, 176.2),
+    (2, 7168, 384, 12, 11.2, 13.1), (8, 7168, 512, 24, 14.0, 14.9), (1, 512, 1024, 4, 9.0, 16.0),
+    (32, 4096, 14336, 30, 357.3, 393.1), (32, 4096, 14336, 34, 367.9, 336.2), (32, 4096, 14336, 48, 386.0, 338.9),
+    (64, 4096, 14336, 48, 775.7, 671.9), (64, 4096, 6400, 30, 338.7, 357.4), (64, 4096, 6400, 40, 347.5, 315.9),
+    (26, 4096, 14336, 37, 333.3, 404.5), (16, 12800, 4096, 48, 195.3, 197.4), (8, 28672, 4096, 48, 190.7, 208.9),
+    (8, 4096, 14336, 6, 84.2, 112.8), (64, 2048, 4096, 48, 128.6, 141.5), (64, 2816, 2048, 48, 91.5, 98.0),
+    (512, 2048, 4096, 32, 912.0, 816.0), (512, 4096, 1024, 24, 477.0, 496.0), (512, 2048, 4096, 1, 468.0, 2348.0),
+]
+
+
+@pytest.mark.parametrize("groups,N,K,rows,stream,other", STREAM)
+def test_streaming_where_it_is_faster(rules, groups, N, K, rows, stream, other):
+    assert (rules.stream_rows(groups * rows, N, K // 128, groups, 256) != 0) == (stream < other)
+
+
+def test_streaming_pass_for_skewed_groups(rules):
+    """Large matrices take a pass of twice the average group's rows or more, so that a few long groups do not stream them
+    several times (8 x [28672, 4096], 64 rows in one group: 71 us at 16 rows a pass, 41 at 32); 16 - 64 rows always."""
+    assert [rules.stream_rows(8 * n, 28672, 32, 8, 256) for n in (1, 4, 5, 8, 16, 24, 25, 48, 49)] == [16, 16, 32, 32, 32, 32, 64, 64, 0]
+    assert [rules.stream_rows(n, 6400, 32, 1, 256) for n in (1, 5, 16, 17, 24, 25, 48, 49)] == [16, 16, 16, 32, 32, 64, 64, 0]
+    assert [rules.stream_rows(64 * n, 2816, 16, 64, 256) for n in (1, 8, 9, 24, 25, 48, 49)] == [16, 16, 32, 32, 64, 64, 0]
+    assert [rules.stream_rows(128 * n, 2816, 16, 128, 256) for n in (1, 8, 9, 24, 25)] == [16, 16, 32, 32, 0]

@@ -46,8 +46,11 @@ CASES = [
     ([3, 5], 256, 512),
     ([0, 17, 1, 0], 256, 384),                                   # three K-blocks: the last step holds one
     ([1, 0, 2, 33, 16, 7, 0, 40], 1024, 4096),                   # items cut into parts; 1, 2, 16, 33 rows
-    ([5, 0, 70], 264, 128),                                      # one K-block; N ends inside an item
-    ([0, 0, 0, 1], 128, 128),                                    # one step in all
+    ([5, 0, 70], 264, 128),                                      # one K-block; N ends inside a tile (the persistent kernel's, few groups)
+    ([5, 0, 70] + [1, 2, 0] * 4, 264, 128),                      # one K-block and more groups: items of one step; N ends inside an item
+    ([0, 0, 0, 1], 128, 128),
+    ([0] * 9 + [1] + [0] * 3, 128, 128),                         # one step in all
+    ([2, 0, 40], 33000, 256),                                    # few groups, but more than one round of tiles
     ([9, 9, 1, 30, 60, 2, 0, 1], 2144, 7168),
     ([48, 64, 32, 16, 65, 1, 0, 47], 512, 1152),                 # 64-row passes, nine K-blocks
     ([i % 5 for i in range(64)], 512, 1024),
