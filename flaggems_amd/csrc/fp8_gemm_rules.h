@@ -51,16 +51,16 @@ inline bool tall_tiles_pay(bool block_scales, int64_t M, int64_t N, int64_t k_bl
 //     and the exchange behind it cost 2 - 5 us more than they save, up to about a dozen groups, whose table the persistent kernel
 //     scans as quickly.  K = 256: 2 x 7168: 1: 12.7 / 10.5   48: 16.8 / 12.3; 8 x 2048: 1: 13.4 / 11.3.  (K = 384: 2 x 7168: 1: 10.8 / 11.6;
 //     K = 256, 16 x 2048: 1: 13.4 / 15.7; 8 x 16384, two rounds: 1: 13.0 / 20.1.)
-// A pass of 16 rows streams fastest (4 stages in flight), 32 are 1 - 3 % slower; 64 another 3 - 9 %.  Where one group holds every row
+// A pass of 16 rows streams fastest (4 stages in flight), 32 are 1 - 3 % slower, 64 another 3 - 9 %.  Where one group holds every row
 // the passes repeat: 8 x [28672, 4096], 64 rows, 16 a pass 71, 32 a pass 41, persistent 41.  So large matrices, whose passes cost
-// most and where the wider pass costs least (8 x [4096, 14336], 64 rows: 84.6 and 84.8 spread evenly, 93 and 88 with unequal groups),
-// take 32 rows from 4 a group on (from 17 rows in all: 1 x [4096, 6400], 5 rows: 15.1 with 16 a pass, 16.7 with 32).  With
-// everything in one group the kernel stays up to 1.8 times slower than the persistent one on large matrices (64 x [4096, 14336],
-// 1024 rows: 253 / 144); spread as routers spread them it is faster.
+// most, take 32 rows from 6 a group on, where groups as unequal as routers make them do not lose by it (8 x [4096, 14336], 64 rows:
+// 84.6 with 16 a pass and 84.8 with 32 spread evenly, 93 and 88 unequal; 8 x [28672, 4096] with [4096, 14336] behind it, 48 rows: 254
+// and 256).  With everything in one group the kernel stays up to 1.9 times slower than the persistent one on large matrices (16 x
+// [28672, 4096], 96 rows: 103 / 54; 64 x [4096, 14336], 1024 rows: 253 / 144); spread as routers spread them it is faster.
 inline int grouped_stream_pass_rows(int64_t M, int64_t N, int64_t k_blocks, int64_t groups, int64_t cus) {
   const bool large = N * k_blocks * 128 >= 24000000;
   if (k_blocks <= 2 && groups * ((N + 255) / 256) <= cus && groups <= (k_blocks == 1 || M > 24 * groups ? 12 : 8)) return 0;
-  if (M <= 16 || M <= (large ? 4 : 8) * groups) return 16;
+  if (M <= 16 || M <= (large ? 6 : 8) * groups) return 16;
   if (M <= 24 * groups) return 32;
   if (M <= 32 * groups) return groups <= 64 ? 64 : 0;
   return M <= 48 * groups && groups <= (large ? 31 : 64) ? 64 : 0;
