@@ -1255,6 +1255,9 @@ extern "C" size_t fg_grouped_block_fp8_gemm_workspace_bytes(int64_t M, int64_t N
   (void)N;
   return fg::grouped_workspace_bytes(M, K);
 }
+extern "C" size_t fg_grouped_block_fp8_gemm_gathered_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t a_rows, int64_t n_groups) {
+  return fg::grouped_gathered_workspace_bytes(M, N, K, a_rows, n_groups);
+}
 
 extern "C" int fg_grouped_block_fp8_gemm(const void* A, int64_t lda,
                                          const void* B, int64_t ldb, int64_t b_group_stride,

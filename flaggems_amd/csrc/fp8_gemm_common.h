@@ -283,7 +283,8 @@ struct GroupedGemm {
 int grouped_stream_rows(const GemmArgs& a, const GroupedGemm& grouped);
 int launch_grouped_stream(const GemmArgs& a, const GroupedGemm& grouped, int rows, void* workspace, size_t workspace_bytes, hipStream_t stream);
 int launch_grouped(const GemmArgs& a, const GroupedGemm& grouped, void* workspace, size_t workspace_bytes, hipStream_t stream);
-// workspace that lets launch_grouped read row-major activation scales from a transposed copy
+// workspace that launch_grouped can use: for rows in sorted order, and for rows read through an index
 size_t grouped_workspace_bytes(int64_t M, int64_t K);
+size_t grouped_gathered_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t a_rows, int64_t n_groups);
 
 }  // namespace fg

@@ -50,6 +50,7 @@
 // round of the grid are cut along K so that every compute unit streams to the end (finish_cut_tile).
 
 #include "fp8_gemm_mfma.h"
+#include "fp8_gemm_rules.h"
 #include <mutex>
 
 namespace fg {
@@ -1053,7 +1054,7 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint8_t* __restr
 constexpr size_t kMaxGatheredBytes = (size_t)1 << 30;
 size_t gathered_bytes(int64_t M, int64_t K) { return (size_t)((M * K + 255) / 256 * 256); }
 bool gather_copy_pays(int64_t M, int64_t K, int64_t tiles, int cus) {
-  return gathered_bytes(M, K) <= kMaxGatheredBytes && (double)tiles / cus * 6.0 > 5.0 + (double)M * (double)K * 2 / 5e6;
+  return M >= 1024 && gathered_bytes(M, K) <= kMaxGatheredBytes && (double)tiles / cus * 6.0 > 5.0 + (double)M * (double)K * 2 / 5e6;
 }
 
 // Tile rows of a grouped problem (PpArgs::tile_rows).  One block: the group ends, forced into ascending order and into
@@ -1198,33 +1199,35 @@ int allow_full_lds(void (*kern)(PpArgs)) {
   return FG_OK;
 }
 
+// Grouped problems with few rows per segment take tiles of 64 or 128 rows (the JN = 1 and 2 instantiations).  The
+// host sees only the average; a segment longer than a tile reads its weights once per tile, and where the tiles
+// are few (at most half the compute units when every segment has one) a longer segment also costs a round of its
+// own, so those take the next tile height sooner.  Measured on 8 segments, [28672, 4096] | [4096, 14336] weights
+// each (896 | 128 tiles), us for 256- / 64- / 128-row tiles by rows a segment on average:
+//    16: 333 222 249 | 203 112 125     32: 295 223 240 | 207 170 128     64: 303 295 243 | 222 178 192
+//    96: 303 336 288 | 219 181 189    128: 293 415 318 | 202 217 182     256: 404 705 463 | 213 351 269
+int grouped_short_jn(int64_t M, int64_t N, int64_t E) {
+  const bool few_tiles = E * ceil_div(N, kBN) * 2 <= cu_count();
+  if (M <= 16 * E) return 1;
+  if (M <= 32 * E) return few_tiles ? 2 : 1;
+  if (M <= 96 * E) return 2;
+  return M <= 128 * E && few_tiles ? 2 : 0;
+}
+// tile rows of a grouped problem at most: every segment ends with at most one tile that is not full
+int64_t grouped_tile_rows_bound(int64_t M, int64_t E, int short_jn) {
+  const int64_t bound = M / (short_jn != 0 ? kShortTileRows * short_jn : kBM) + E;
+  return bound < M ? bound : M;
+}
+
 int launch_block(const GemmArgs& g, int mode, void* workspace, size_t workspace_bytes, hipStream_t stream,
                  const GroupedGemm* grouped = nullptr) {
   PpArgs a = {};
   a.g = g;
   a.g.tiles_m = (int)ceil_div(g.M, kBM);
-  // Grouped problems with few rows per segment take tiles of 64 or 128 rows (the JN = 1 and 2 instantiations).  The
-  // host sees only the average; a segment longer than a tile reads its weights once per tile, and where the tiles
-  // are few (at most half the compute units when every segment has one) a longer segment also costs a round of its
-  // own, so those take the next tile height sooner.  Measured on 8 segments, [28672, 4096] | [4096, 14336] weights
-  // each (896 | 128 tiles), us for 256- / 64- / 128-row tiles by rows a segment on average:
-  //    16: 333 222 249 | 203 112 125     32: 295 223 240 | 207 170 128     64: 303 295 243 | 222 178 192
-  //    96: 303 336 288 | 219 181 189    128: 293 415 318 | 202 217 182     256: 404 705 463 | 213 351 269
-  int short_jn = 0;
-  if (grouped != nullptr) {
-    const int64_t E = grouped->n_groups;
-    const bool few_tiles = E * ceil_div(g.N, kBN) * 2 <= cu_count();
-    if (g.M <= 16 * E) short_jn = 1;
-    else if (g.M <= 32 * E) short_jn = few_tiles ? 2 : 1;
-    else if (g.M <= 96 * E) short_jn = 2;
-    else if (g.M <= 128 * E) short_jn = few_tiles ? 2 : 0;
-  }
+  const int short_jn = grouped != nullptr ? grouped_short_jn(g.M, g.N, grouped->n_groups) : 0;
   const bool short_tiles = short_jn != 0;
   if (grouped != nullptr) {
-    // every segment ends with at most one tile that is not full; the kernel counts the real tiles
-    const int tile_rows = short_tiles ? kShortTileRows * short_jn : kBM;
-    const int64_t bound = g.M / tile_rows + grouped->n_groups;
-    a.g.tiles_m = (int)(bound < g.M ? bound : g.M);
+    a.g.tiles_m = (int)grouped_tile_rows_bound(g.M, grouped->n_groups, short_jn);  // (the kernel counts the real ones)
     a.groups = grouped->ends; a.n_groups = (int)grouped->n_groups;
     a.w_group_stride = grouped->w_group_stride; a.ws_group_stride = grouped->ws_group_stride;
     a.row_index = grouped->row_index; a.index_div = (int)grouped->index_div; a.x_rows = (int)grouped->x_rows;
@@ -1265,22 +1268,23 @@ int launch_block(const GemmArgs& g, int mode, void* workspace, size_t workspace_
   const size_t need = FG_WORKSPACE_COUNTER_BYTES + sk_bytes;
   // rows of the activation-scale matrix: the rows of X, which a gathered problem reads through its index
   const int64_t scale_rows = (grouped != nullptr && grouped->row_index != nullptr && grouped->index_div > 0) ? grouped->x_rows : (int64_t)g.M;
-  // workspace: [counters][partial tiles, if the shape is one that shares tiles][transposed activation scales]
+  // workspace: [counters][partial tiles, if the shape is one that shares tiles][transposed activation scales][rows of a gathered
+  // problem][table of tile rows], each where the launch has it
   // (a grouped problem's tile count is an upper bound that a few hundred rows spread over many segments inflate:
   // there the gathers are few and the transposition, ~5 us whatever the size, does not pay)
-  size_t at = need + transposed_scales_bytes(scale_rows > g.M ? scale_rows : g.M, g.KB);  // what follows the scales
+  size_t at = need;
   if (a.gather_index != nullptr && !short_tiles && workspace != nullptr && (uintptr_t)workspace % 16 == 0 && g.K % 128 == 0 &&
       g.ldx % 16 == 0 && (uintptr_t)g.X % 16 == 0 && gather_copy_pays(g.M, g.K, tiles, cus) &&
-      workspace_bytes >= at + gathered_bytes(g.M, g.K)) {
+      workspace_bytes >= need + transposed_scales_bytes(g.M, g.KB) + gathered_bytes(g.M, g.K)) {
     float* const xs_t = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + need);
-    uint8_t* const rows = reinterpret_cast<uint8_t*>(workspace) + at;
+    uint8_t* const rows = reinterpret_cast<uint8_t*>(workspace) + need + transposed_scales_bytes(g.M, g.KB);
     FG_LAUNCH(gather_rows_kernel, dim3((uint32_t)ceil_div(g.M, kGatherRows)), dim3(256), 0, stream, g.X, g.ldx, g.xs, g.xs_rs, g.xs_cs, a.row_index,
               a.index_div, a.x_rows, g.M, g.K, rows, xs_t);
     FG_CHECK_LAUNCH("gather_rows_kernel");
     a.g.X = rows; a.g.ldx = g.K;
     a.g.xs = xs_t; a.g.xs_rs = 1; a.g.xs_cs = g.M;
     a.gather_index = nullptr;
-    at += gathered_bytes(g.M, g.K);
+    at += transposed_scales_bytes(g.M, g.KB) + gathered_bytes(g.M, g.K);
   } else if (mode == kModeBlock && g.xs_rs >= kTransposeMinRowStride && transposition_pays(tiles, g.KB, cus) && workspace != nullptr &&
       (grouped == nullptr || g.M >= 1024) &&
       (uintptr_t)workspace % 16 == 0 &&
@@ -1290,6 +1294,7 @@ int launch_block(const GemmArgs& g, int mode, void* workspace, size_t workspace_
                        dim3(256), 0, stream, g.xs, g.xs_rs, g.xs_cs, (int)scale_rows, g.KB, xs_t);
     FG_CHECK_LAUNCH("transpose_scales_kernel");
     a.g.xs = xs_t; a.g.xs_rs = 1; a.g.xs_cs = scale_rows;
+    at += transposed_scales_bytes(scale_rows, g.KB);
   }
   if (grouped != nullptr && a.n_groups * (tiles > cus ? tiles / cus : 1) >= kTableMinScans && a.n_groups <= kTableGroups && workspace != nullptr) {
     if ((uintptr_t)workspace % 16 == 0 && workspace_bytes >= at + tile_table_bytes(a.g.tiles_m)) {
@@ -1388,10 +1393,20 @@ size_t pingpong_workspace_bytes(int64_t M, int64_t N, int64_t K) {
 
 size_t grouped_workspace_bytes(int64_t M, int64_t K) {
   if (M <= 0 || K <= 0 || K % 128 != 0) return 0;
-  // (the partial sums of cut short tiles: the number of segments is not known here, the bound of the plan is)
-  return FG_WORKSPACE_COUNTER_BYTES + (size_t)kMaxCutItems * kCutSlotBytes + transposed_scales_bytes(M, K / 128) +
-         tile_table_bytes(M) +  // (a tile row holds at least one row)
-         (M >= 1024 && gathered_bytes(M, K) <= kMaxGatheredBytes ? gathered_bytes(M, K) : 0);
+  // (the partial sums of cut tiles and the table: the number of segments is not known here, the bound of the plan is, and a tile
+  // row holds at least one row)
+  return FG_WORKSPACE_COUNTER_BYTES + (size_t)kMaxCutItems * kCutSlotBytes + transposed_scales_bytes(M, K / 128) + tile_table_bytes(M);
+}
+
+// The same for rows read through an index: the scales are those of a_rows rows, unless the rows are copied first.
+size_t grouped_gathered_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t a_rows, int64_t E) {
+  if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || a_rows <= 0 || E <= 0) return 0;
+  const int64_t KB = K / 128;
+  const int short_jn = grouped_short_jn(M, N, E);
+  const int64_t tiles = grouped_tile_rows_bound(M, E, short_jn) * ceil_div(N, (int64_t)kBN);
+  const bool copied = grouped_stream_pass_rows(M, N, KB, E, cu_count()) == 0 && short_jn == 0 && gather_copy_pays(M, K, tiles, cu_count());
+  return FG_WORKSPACE_COUNTER_BYTES + (size_t)kMaxCutItems * kCutSlotBytes + tile_table_bytes(M) +
+         (copied ? transposed_scales_bytes(M, KB) + gathered_bytes(M, K) : transposed_scales_bytes(a_rows, KB));
 }
 
 int launch_grouped(const GemmArgs& g, const GroupedGemm& grouped, void* workspace, size_t workspace_bytes, hipStream_t stream) {

@@ -164,7 +164,10 @@ def grouped_w8a8_block_fp8_matmul(
     lib = _lib.load()
     dev = A.device
     with _lib.device_guard(dev):
-        ws_bytes = _lib.cached_workspace_bytes("fg_grouped_block_fp8_gemm_workspace_bytes", max(M, T), N, K)
+        if row_index is not None and index_divisor > 0:
+            ws_bytes = _lib.cached_workspace_bytes("fg_grouped_block_fp8_gemm_gathered_workspace_bytes", M, N, K, T, E)
+        else:
+            ws_bytes = _lib.cached_workspace_bytes("fg_grouped_block_fp8_gemm_workspace_bytes", M, N, K)
         ws = _lib.workspace(dev, ws_bytes) if ws_bytes else None
         status = lib.fg_grouped_block_fp8_gemm(
             A.data_ptr(), A.stride(0) if T > 1 else max(K, A.stride(0)),

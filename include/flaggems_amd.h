@@ -418,10 +418,14 @@ int fg_batched_block_fp8_gemm(const void* A, int64_t lda, int64_t a_batch_stride
  * K must be a positive multiple of 128; A, B 16-byte aligned with lda, ldb, b_group_stride multiples of 16;
  * C 16-byte aligned with ldc a multiple of 8; c_dtype FG_BF16 or FG_F16 (FG_ERR_UNSUPPORTED otherwise: there is no
  * slower general path behind this entry point).
- * `workspace` (optional, 16-byte aligned, fg_grouped_block_fp8_gemm_workspace_bytes(M, N, K) bytes, first
- * FG_WORKSPACE_COUNTER_BYTES zero-filled once) lets row-major As be read from a transposed copy and, when the
- * groups average at most 128 rows (M <= 128 * n_groups), lets tiles be cut along K so that few tiles fill the GPU
- * (64 MB of partial sums; the sums are added in a fixed order, but not in the order of the call without workspace).
+ * `workspace` (optional, 16-byte aligned, first FG_WORKSPACE_COUNTER_BYTES zero-filled once) holds, each where the
+ * launch has it: partial sums (64 MB), so that tiles are cut along K and items shared where few of them would leave
+ * compute units idle (added in a fixed order, but not in the order of the call without workspace); row-major As
+ * transposed (4 * rows * K / 128 bytes); with row_index and large problems, the rows of A in sorted order (M * K bytes,
+ * at most 1 GiB); with many groups, a table of tile rows (16 * (M + 1) bytes at most).  An area that does not fit is
+ * done without.  What a call can use: fg_grouped_block_fp8_gemm_workspace_bytes(M, N, K) with rows in sorted order
+ * (row_index NULL or index_div 0), fg_grouped_block_fp8_gemm_gathered_workspace_bytes(M, N, K, a_rows, n_groups) with
+ * rows read through row_index.
  * row_index (optional DEVICE table of M int32): the kernel gathers its rows itself -- row m of the sorted order
  * (the order of group_ends and of C) is row row_index[m] / index_div of A and As, which then have a_rows rows
  * (entries are forced into [0, a_rows); a_rows * lda must fit 32 bits).  This is how the reference's MoE kernel
@@ -454,6 +458,7 @@ int fg_grouped_block_fp8_gemm(const void* A, int64_t lda,
                               int64_t M, int64_t N, int64_t K, int64_t block_n, int64_t block_k,
                               void* workspace, size_t workspace_bytes, void* stream);
 size_t fg_grouped_block_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K);
+size_t fg_grouped_block_fp8_gemm_gathered_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t a_rows, int64_t n_groups);
 
 /*
  * Per-tensor / per-token x per-channel scaled FP8 GEMM with optional bias:

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import flag_gems
+from flaggems_amd import _lib
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -48,3 +49,45 @@ def test_rows_copied_in_sorted_order(T, M, N, K, E, top_k, column_major):
             # half a bf16 step, plus the matrix instruction's alignment of 128 products to the largest one
             assert ((got[begin:end].float() - want).abs() <= want.abs() * 2.0 ** -8 + 4e-4 * mag).all()
         begin = end
+
+
+@pytest.mark.parametrize("T,M,N,K,E,sums", [(4096, 1040, 8448, 256, 5, 0), (2048, 4096, 6144, 2048, 24, 64)])
+def test_workspace_of_the_stated_size_is_enough(T, M, N, K, E, sums):
+    """Workspace of exactly fg_grouped_block_fp8_gemm_gathered_workspace_bytes: the rows are copied (they lie behind the counters, the
+    partial sums, where K is long enough to be cut, and their scales), nothing is written past its end, and the results are those of the public call."""
+    x, w, xs, ws, ends, g = _problem(T, M, N, K, E, M + N, False)
+    idx = torch.randint(0, T, (M,), generator=g, device=DEV).int()
+    lib = _lib.load()
+    size = lib.fg_grouped_block_fp8_gemm_gathered_workspace_bytes(M, N, K, T, E)
+    work = torch.zeros(size + 4096, dtype=torch.uint8, device=DEV)
+    work[size:] = 0xA5
+    c = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    status = lib.fg_grouped_block_fp8_gemm(
+        x.data_ptr(), K, w.data_ptr(), K, N * K, xs.data_ptr(), xs.stride(0), xs.stride(1), ws.data_ptr(), ws.stride(1), 1, ws.stride(0),
+        ends.data_ptr(), E, idx.data_ptr(), 1, T, 0, None, c.data_ptr(), N, _lib.DTYPE_CODE[torch.bfloat16], M, N, K, 128, 128,
+        work.data_ptr(), size, _lib.current_stream_ptr(torch.device(DEV)))
+    _lib.check(status, "fg_grouped_block_fp8_gemm")
+    at = _lib.FG_WORKSPACE_COUNTER_BYTES + (sums << 20) + -(-4 * M * (K // 128) // 256) * 256
+    rows = work[at:at + M * K].view(M, K)
+    assert torch.equal(rows, x[idx.long()].view(torch.uint8))
+    assert (work[size:] == 0xA5).all()
+    same = flag_gems.grouped_w8a8_block_fp8_matmul(x, w, xs, ws, ends, [128, 128], row_index=idx)
+    last = int(ends[-1])
+    assert torch.equal(c[:last], same[:last])
+
+
+@pytest.mark.parametrize("divisor", [None, 0, 2])
+def test_only_gathered_calls_ask_for_the_copy(divisor, monkeypatch):
+    M, N, K, E = 1024, 256, 512, 2
+    T = M // 2 if divisor == 2 else M
+    x, w, xs, ws, ends, g = _problem(T, M, N, K, E, 7, False)
+    idx = None if divisor is None else torch.randperm(M, generator=g, device=DEV).int()
+    asked = []
+    real = _lib.cached_workspace_bytes
+    monkeypatch.setattr(_lib, "cached_workspace_bytes", lambda name, *shape: asked.append((name, shape)) or real(name, *shape))
+    flag_gems.grouped_w8a8_block_fp8_matmul(x, w, xs, ws, ends, [128, 128], row_index=idx, index_divisor=1 if divisor is None else divisor,
+                                            scatter_rows=None if divisor is None else M)
+    if divisor:
+        assert asked == [("fg_grouped_block_fp8_gemm_gathered_workspace_bytes", (M, N, K, T, E))]
+    else:
+        assert asked == [("fg_grouped_block_fp8_gemm_workspace_bytes", (M, N, K))]
