@@ -1048,14 +1048,7 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const uint8_t* __restr
     for (int kb = tid / kGatherRows; kb < (K >> 7); kb += 256 / kGatherRows)
       out_scales[(int64_t)kb * M + m0 + r] = xs[(int64_t)s_src[r] * rs + (int64_t)kb * cs];
 }
-// Where it pays.  Reading 256-row tiles through the index costs a block about 10 us at every tile: index loads and their
-// divisions, whose waits cover every copy in flight, in two walks.  The copy moves 2 M K bytes once and is a launch (4096
-// tokens twice, K = 4096: 12 us); 8192 rows, 8 segments, [28672, 4096], 15.8 tiles a block: GEMM 1212 -> 1041 us.
-constexpr size_t kMaxGatheredBytes = (size_t)1 << 30;
 size_t gathered_bytes(int64_t M, int64_t K) { return (size_t)((M * K + 255) / 256 * 256); }
-bool gather_copy_pays(int64_t M, int64_t K, int64_t tiles, int cus) {
-  return M >= 1024 && gathered_bytes(M, K) <= kMaxGatheredBytes && (double)tiles / cus * 6.0 > 5.0 + (double)M * (double)K * 2 / 5e6;
-}
 
 // Tile rows of a grouped problem (PpArgs::tile_rows).  One block: the group ends, forced into ascending order and into
 // [0, M] as segment_end does, and the tile rows before every group by scans in LDS; then every tile row finds its group
@@ -1115,7 +1108,8 @@ __global__ __launch_bounds__(1024) void group_tile_rows_kernel(const int* ends, 
 constexpr int kShortTileRows = 64;
 constexpr size_t kCutSlotBytes = (size_t)8 * kTN * 256 * 4;  // a work item's partial sums: 8 wavefronts x 16 x 128 floats
 // A launch of one block, about 5 us, against a scan of about 0.1 us a group in each of three walks at every tile a block
-// enters: from some two dozen (groups x tiles a block) on.  8 groups, 15.8 tiles a block (8192 rows, [28672, 4096]): 1243 -> 1212 us.
+// enters.  4000 random problems by groups x tiles a block, with the table / without: 8: 1.02, 11: 1.00, 16: 0.97, 23: 0.92, 45: 0.84,
+// 256: 0.64, 1000: 0.5; from 24 on at most 4 % slower.  8 groups, 15.8 tiles a block (8192 rows, [28672, 4096]): 1243 -> 1212 us.
 constexpr int64_t kTableMinScans = 24;
 size_t tile_table_bytes(int64_t tile_rows) { return (size_t)(tile_rows + 1) * sizeof(int4); }
 // Largest number of cuts per tile of the last round, as a shift (the kernel picks among 0..this from the real tile
@@ -1274,7 +1268,7 @@ int launch_block(const GemmArgs& g, int mode, void* workspace, size_t workspace_
   // there the gathers are few and the transposition, ~5 us whatever the size, does not pay)
   size_t at = need;
   if (a.gather_index != nullptr && !short_tiles && workspace != nullptr && (uintptr_t)workspace % 16 == 0 && g.K % 128 == 0 &&
-      g.ldx % 16 == 0 && (uintptr_t)g.X % 16 == 0 && gather_copy_pays(g.M, g.K, tiles, cus) &&
+      g.ldx % 16 == 0 && (uintptr_t)g.X % 16 == 0 && gather_copy_pays(g.M, g.N, g.K, grouped->n_groups, cus) &&
       workspace_bytes >= need + transposed_scales_bytes(g.M, g.KB) + gathered_bytes(g.M, g.K)) {
     float* const xs_t = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + need);
     uint8_t* const rows = reinterpret_cast<uint8_t*>(workspace) + need + transposed_scales_bytes(g.M, g.KB);
@@ -1403,8 +1397,7 @@ size_t grouped_gathered_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 != 0 || a_rows <= 0 || E <= 0) return 0;
   const int64_t KB = K / 128;
   const int short_jn = grouped_short_jn(M, N, E);
-  const int64_t tiles = grouped_tile_rows_bound(M, E, short_jn) * ceil_div(N, (int64_t)kBN);
-  const bool copied = grouped_stream_pass_rows(M, N, KB, E, cu_count()) == 0 && short_jn == 0 && gather_copy_pays(M, K, tiles, cu_count());
+  const bool copied = grouped_stream_pass_rows(M, N, KB, E, cu_count()) == 0 && short_jn == 0 && gather_copy_pays(M, N, K, E, cu_count());
   return FG_WORKSPACE_COUNTER_BYTES + (size_t)kMaxCutItems * kCutSlotBytes + tile_table_bytes(M) +
          (copied ? transposed_scales_bytes(M, KB) + gathered_bytes(M, K) : transposed_scales_bytes(a_rows, KB));
 }

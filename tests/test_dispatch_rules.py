@@ -14,6 +14,7 @@ extern "C" int tall(int block, long long M, long long N, long long kb, long long
 extern "C" int stream_rows(long long M, long long N, long long kb, long long groups, long long cus) {
   return fg::grouped_stream_pass_rows(M, N, kb, groups, cus);
 }
+extern "C" int copy_rows(long long M, long long N, long long K, long long groups, long long cus) { return fg::gather_copy_pays(M, N, K, groups, cus); }
 """ % HEADER
 
 
@@ -29,7 +30,7 @@ def rules(tmp_path_factory):
     subprocess.run([cxx, "-std=c++17", "-O1", "-Wall", "-Werror", "-shared", "-fPIC", "-o", lib, src], check=True)
     so = ctypes.CDLL(lib)
     so.tall.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
-    so.stream_rows.argtypes = [ctypes.c_longlong] * 5
+    so.stream_rows.argtypes = so.copy_rows.argtypes = [ctypes.c_longlong] * 5
     return so
 
 
@@ -90,3 +91,18 @@ def test_streaming_pass_for_skewed_groups(rules):
     assert [rules.stream_rows(n, 6400, 32, 1, 256) for n in (1, 5, 16, 17, 24, 25, 48, 49)] == [16, 16, 16, 32, 32, 64, 64, 0]
     assert [rules.stream_rows(64 * n, 2816, 16, 64, 256) for n in (1, 8, 9, 24, 25, 48, 49)] == [16, 16, 32, 32, 64, 64, 0]
     assert [rules.stream_rows(128 * n, 2816, 16, 128, 256) for n in (1, 8, 9, 24, 25)] == [16, 16, 32, 32, 0]
+
+
+# groups, N, K, rows, us with the gathered rows copied first, us read through the index
+COPY = [
+    (8, 28672, 4096, 1118, 266.2, 319.5), (8, 28672, 4096, 7825, 918.0, 1201.3), (6, 12800, 4096, 2020, 143.3, 170.5),
+    (6, 4096, 1024, 4071, 50.6, 56.7), (8, 4096, 1024, 4203, 51.6, 57.7), (1, 12800, 4096, 2099, 114.0, 131.6),
+    (3, 12800, 4096, 782, 71.8, 82.1), (2, 30016, 7296, 322, 127.0, 151.0),
+    (8, 7168, 256, 1139, 24.0, 20.9), (6, 5888, 128, 2267, 21.0, 18.1), (16, 1024, 256, 13882, 28.0, 23.6), (1, 7168, 256, 1787, 22.1, 20.0),
+    (6, 1408, 128, 8325, 23.2, 19.9), (2, 1536, 128, 13798, 29.6, 27.0), (2, 3456, 128, 8229, 31.3, 29.2), (64, 576, 256, 10833, 27.4, 24.5),
+]
+
+
+@pytest.mark.parametrize("groups,N,K,rows,copied,indexed", COPY)
+def test_gathered_rows_are_copied_where_that_is_faster(rules, groups, N, K, rows, copied, indexed):
+    assert bool(rules.copy_rows(rows, N, K, groups, 256)) == (copied < indexed)

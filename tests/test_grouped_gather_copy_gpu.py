@@ -30,6 +30,12 @@ def _problem(T, M, N, K, E, seed, column_major):
     (200, 1205, 8200, 384, 4, 6, False),     # three K-blocks, more than one row of the sixteen from the same token
     (4096, 1040, 8448, 256, 5, 1, False),    # more source rows than sorted ones
     (2048, 4096, 6144, 2048, 24, 2, False),  # table of tile rows
+    # the first four read through the index (one round of tiles); the same edges where the rows are copied
+    (550, 1100, 16400, 256, 3, 2, False),
+    (1100, 1100, 28704, 128, 3, 1, True),
+    (200, 1205, 16400, 384, 4, 6, False),
+    (4096, 1040, 16640, 256, 5, 1, False),
+    (150, 300, 32776, 384, 2, 2, False),     # few rows, many tiles
 ])
 def test_rows_copied_in_sorted_order(T, M, N, K, E, top_k, column_major):
     x, w, xs, ws, ends, g = _problem(T, M, N, K, E, M + N + K, column_major)
@@ -51,7 +57,7 @@ def test_rows_copied_in_sorted_order(T, M, N, K, E, top_k, column_major):
         begin = end
 
 
-@pytest.mark.parametrize("T,M,N,K,E,sums", [(4096, 1040, 8448, 256, 5, 0), (2048, 4096, 6144, 2048, 24, 64)])
+@pytest.mark.parametrize("T,M,N,K,E,sums", [(4096, 1040, 16640, 256, 5, 0), (2048, 4096, 6144, 2048, 24, 64)])
 def test_workspace_of_the_stated_size_is_enough(T, M, N, K, E, sums):
     """Workspace of exactly fg_grouped_block_fp8_gemm_gathered_workspace_bytes: the rows are copied (they lie behind the counters, the
     partial sums, where K is long enough to be cut, and their scales), nothing is written past its end, and the results are those of the public call."""

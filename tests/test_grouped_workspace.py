@@ -34,12 +34,13 @@ def test_rows_in_sorted_order_ask_for_no_copy(M, N, K):
 
 @pytest.mark.parametrize("M,N,K,a_rows,groups,copied", [
     (8192, 28672, 4096, 4096, 8, True),      # Mixtral's gate/up product on 4096 tokens
-    (1040, 8448, 256, 4096, 5, True),        # more source rows than sorted ones
-    (1040, 8448, 256, 300, 5, True),
-    (1023, 28672, 4096, 512, 3, False),      # below the copy's rule
+    (1040, 16640, 256, 4096, 5, True),       # more source rows than sorted ones
+    (1040, 16640, 256, 300, 5, True),
+    (1040, 8448, 256, 4096, 5, False),       # one round of tiles
+    (500, 28672, 4096, 512, 2, True),        # few rows, many tiles
     (1024, 28672, 4096, 512, 16, False),     # 64 rows a group: 128-row tiles read through the index
     (300, 28672, 4096, 150, 8, False),       # streaming kernel
-    (2048, 512, 4096, 1024, 4, False),       # too few tiles for a copy to pay
+    (2048, 512, 4096, 1024, 4, False),
     (300000, 28672, 4096, 150000, 8, False),  # over 1 GiB
 ])
 def test_gathered_rows(M, N, K, a_rows, groups, copied):
