@@ -540,16 +540,15 @@ __global__ __launch_bounds__(WM* WN * 64) void fp8_gemm_kernel(GemmArgs a) {
     if (lane == 0) prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     prev = (unsigned int)__builtin_amdgcn_readfirstlane((int)prev);
     if (prev != (unsigned int)(a.splits - 1)) return;
-    // The parts of a batch are in flight together: a part at a time costs a round trip to memory each (about 1 us).  A batch
-    // that runs past the last part would read that one again and leave it out of the sum.
+    // The parts of a batch (one, or both of two) are in flight together: a part at a time costs a round trip to memory each
+    // (about 1 us).
     auto add_parts = [&](auto batch) __attribute__((always_inline)) {
       constexpr int kBatch = decltype(batch)::value;
       for (int s0 = 0; s0 < a.splits; s0 += kBatch) {
         v4f tmp[kBatch][TN][TM];
 #pragma unroll
         for (int q = 0; q < kBatch; ++q) {
-          const int s = s0 + q < a.splits ? s0 + q : a.splits - 1;
-          const float* const src = uniform_ptr(a.split_partials + ((size_t)tile_id * a.splits + s) * kSlotFloats);
+          const float* const src = uniform_ptr(a.split_partials + ((size_t)tile_id * a.splits + s0 + q) * kSlotFloats);
 #pragma unroll
           for (int i = 0; i < TN; ++i)
 #pragma unroll
@@ -562,8 +561,7 @@ __global__ __launch_bounds__(WM* WN * 64) void fp8_gemm_kernel(GemmArgs a) {
 #pragma unroll
             for (int j = 0; j < TM; ++j) asm volatile("s_waitcnt vmcnt(0)" : "+v"(tmp[q][i][j]) : : "memory");
 #pragma unroll
-        for (int q = 0; q < kBatch; ++q) {
-          if (s0 + q >= a.splits) break;
+        for (int q = 0; q < kBatch; ++q)
 #pragma unroll
           for (int i = 0; i < TN; ++i)
 #pragma unroll
@@ -573,7 +571,6 @@ __global__ __launch_bounds__(WM* WN * 64) void fp8_gemm_kernel(GemmArgs a) {
               else if (MODE == kModeRowColI8) acc[i][j] = __builtin_bit_cast(v4f, __builtin_bit_cast(v4i, acc[i][j]) + __builtin_bit_cast(v4i, tmp[q][i][j]));
               else acc[i][j] += tmp[q][i][j];
             }
-        }
       }
     };
     // (only where there are two: in batches of four the registers of a second block on the compute unit are gone, and the

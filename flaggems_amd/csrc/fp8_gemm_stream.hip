@@ -44,7 +44,7 @@ constexpr int kRing = 8;                     // items whose row indices are kept
 
 struct StreamArgs {
   GemmArgs g;
-  // groups (null: one group of M rows): cumulative row ends, forced into ascending order and into [0, M]
+  // groups: cumulative row ends, forced into ascending order and into [0, M]
   const int* ends;
   int n_groups;
   int64_t w_group_stride, ws_group_stride;
@@ -112,7 +112,7 @@ __device__ __forceinline__ int wave_scan_sum(int v, int lane) {
   return v;
 }
 
-template <int TMX, int MODE>
+template <int TMX>
 __global__ __launch_bounds__(kThreads) void fp8_gemm_stream_kernel(StreamArgs a) {
   using C = Cfg<TMX>;
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
@@ -129,15 +129,9 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_stream_kernel(StreamArgs a)
   {
     int* const sums = reinterpret_cast<int*>(lds + C::kIndexOff);  // [2][kWaves], free until the first item
     const int e0 = 2 * tid, e1 = e0 + 1;
-    int v0 = 0, v1 = 0;
-    if (a.ends == nullptr) {
-      v0 = v1 = tid == 0 ? g.M : 0;
-    } else {
-      if (e0 < E) v0 = a.ends[e0];
-      if (e1 < E) v1 = a.ends[e1];
-      v0 = v0 < 0 ? 0 : (v0 < g.M ? v0 : g.M);
-      v1 = v1 < 0 ? 0 : (v1 < g.M ? v1 : g.M);
-    }
+    int v0 = e0 < E ? a.ends[e0] : 0, v1 = e1 < E ? a.ends[e1] : 0;
+    v0 = v0 < 0 ? 0 : (v0 < g.M ? v0 : g.M);
+    v1 = v1 < 0 ? 0 : (v1 < g.M ? v1 : g.M);
     v1 = v1 > v0 ? v1 : v0;
     const int incl = wave_scan_max(v1, lane);
     if (lane == 63) sums[wave] = incl;
@@ -242,7 +236,7 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_stream_kernel(StreamArgs a)
   int64_t s_step = 0;
   const bool odd_k = (g.KB & 1) != 0;
   // waves whose copy carries the weight scales: TMX 4 needs two copies for the activation scales (one per K-block)
-  const bool ws_wave = MODE == kModeBlock && (TMX == 4 ? (wave & 2) != 0 : (wave & 1) != 0);
+  const bool ws_wave = TMX == 4 ? (wave & 2) != 0 : (wave & 1) != 0;
 
   auto copy_index = [&](const Walk& w) __attribute__((always_inline)) {
     if (a.row_index == nullptr) return;
@@ -278,17 +272,15 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_stream_kernel(StreamArgs a)
       const int r = TMX == 1 ? wave * 2 + ((lane >> 4) & 1) : (wave * C::kXCopies + j) * 4 + lg;
       x_off[j] = (uint32_t)source_row(w, r) * (uint32_t)g.ldx + (uint32_t)((l16 ^ (r & 15)) << 4);
     }
-    if (MODE == kModeBlock) {
-      if (ws_wave) {
-        s_base = uniform_ptr(g.ws + (int64_t)w.group * a.ws_group_stride + (int64_t)w.chunk * g.ws_rs);
-        s_off = (uint32_t)(lane & 1) * (uint32_t)g.ws_cs * 4u;
-        s_step = g.ws_cs;
-      } else {
-        s_base = uniform_ptr(g.xs + (gathered ? 0 : (int64_t)m0 * g.xs_rs));
-        const int b = TMX == 4 ? (wave & 1) : (lane >> (TMX == 1 ? 4 : 5)) & 1;
-        s_off = ((uint32_t)source_row(w, lane & (C::kRows - 1)) * (uint32_t)g.xs_rs + (uint32_t)b * (uint32_t)g.xs_cs) * 4u;
-        s_step = g.xs_cs;
-      }
+    if (ws_wave) {
+      s_base = uniform_ptr(g.ws + (int64_t)w.group * a.ws_group_stride + (int64_t)w.chunk * g.ws_rs);
+      s_off = (uint32_t)(lane & 1) * (uint32_t)g.ws_cs * 4u;
+      s_step = g.ws_cs;
+    } else {
+      s_base = uniform_ptr(g.xs + (gathered ? 0 : (int64_t)m0 * g.xs_rs));
+      const int b = TMX == 4 ? (wave & 1) : (lane >> (TMX == 1 ? 4 : 5)) & 1;
+      s_off = ((uint32_t)source_row(w, lane & (C::kRows - 1)) * (uint32_t)g.xs_rs + (uint32_t)b * (uint32_t)g.xs_cs) * 4u;
+      s_step = g.xs_cs;
     }
     if (a.row_weight != nullptr && lane < C::kRows) {
       int idx = ring_index[(w.serial & (kRing - 1)) * 64 + lane];
@@ -301,15 +293,13 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_stream_kernel(StreamArgs a)
     const bool half = odd_k && pair == KP - 1;  // the pair's second K-block does not exist: its pieces repeat the first's
     const uint8_t* const wp = uniform_ptr(w_base + (int64_t)pair * 256);
     const uint8_t* const xp = uniform_ptr(x_base + (int64_t)pair * 256);
-    if (MODE == kModeBlock) {
-      const float* const sp = uniform_ptr(s_base + (int64_t)pair * 2 * s_step);
-      if (ws_wave) {
-        if (lane < 2) copy4(half ? 0u : s_off, sp, stage + kWBytes + C::kXBytes + 2 * C::kRows * 4);
-      } else {
-        const bool second = TMX == 4 ? (wave & 1) != 0 : lane >= C::kRows;
-        const uint32_t off = half && second ? s_off - (uint32_t)g.xs_cs * 4u : s_off;
-        if (TMX > 1 || lane < 32) copy4(off, sp, stage + kWBytes + C::kXBytes + (TMX == 4 ? (uint32_t)(wave & 1) * C::kRows * 4 : 0u));
-      }
+    const float* const sp = uniform_ptr(s_base + (int64_t)pair * 2 * s_step);
+    if (ws_wave) {
+      if (lane < 2) copy4(half ? 0u : s_off, sp, stage + kWBytes + C::kXBytes + 2 * C::kRows * 4);
+    } else {
+      const bool second = TMX == 4 ? (wave & 1) != 0 : lane >= C::kRows;
+      const uint32_t off = half && second ? s_off - (uint32_t)g.xs_cs * 4u : s_off;
+      if (TMX > 1 || lane < 32) copy4(off, sp, stage + kWBytes + C::kXBytes + (TMX == 4 ? (uint32_t)(wave & 1) * C::kRows * 4 : 0u));
     }
 #pragma unroll
     for (int j = 0; j < C::kXCopies; ++j) {
@@ -382,20 +372,16 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_stream_kernel(StreamArgs a)
         return f;
       };
       const v8i wf = fragment(sw);
-      const float wsv = MODE == kModeBlock ? sc[2 * C::kRows + b] : 1.f;
+      const float wsv = sc[2 * C::kRows + b];
 #pragma unroll
       for (int t = 0; t < TMX; ++t) {
         const v8i xf = fragment(sx + t * 4096);
-        if (MODE == kModeBlock) {
-          const float f = sc[b * C::kRows + t * 16 + l16] * wsv;
-          const v4f p = mfma_fp8_16x16x128(wf, xf, v4f{0.f, 0.f, 0.f, 0.f});
-          acc[t][0] = __builtin_fmaf(p[0], f, acc[t][0]);
-          acc[t][1] = __builtin_fmaf(p[1], f, acc[t][1]);
-          acc[t][2] = __builtin_fmaf(p[2], f, acc[t][2]);
-          acc[t][3] = __builtin_fmaf(p[3], f, acc[t][3]);
-        } else {
-          acc[t] = MODE == kModeRowColI8 ? mfma_i8_16x16x128(wf, xf, acc[t]) : mfma_fp8_16x16x128(wf, xf, acc[t]);
-        }
+        const float f = sc[b * C::kRows + t * 16 + l16] * wsv;
+        const v4f p = mfma_fp8_16x16x128(wf, xf, v4f{0.f, 0.f, 0.f, 0.f});
+        acc[t][0] = __builtin_fmaf(p[0], f, acc[t][0]);
+        acc[t][1] = __builtin_fmaf(p[1], f, acc[t][1]);
+        acc[t][2] = __builtin_fmaf(p[2], f, acc[t][2]);
+        acc[t][3] = __builtin_fmaf(p[3], f, acc[t][3]);
       }
     }
     slot = slot + 1 == C::kStages ? 0 : slot + 1;
@@ -434,8 +420,6 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_stream_kernel(StreamArgs a)
 #pragma unroll
           for (int t = 0; t < TMX; ++t) {
             if (b == fb) acc[t] = tmp[t];
-            else if (MODE == kModeRowColI8)
-              acc[t] = __builtin_bit_cast(v4f, __builtin_bit_cast(v4i, acc[t]) + __builtin_bit_cast(v4i, tmp[t]));
             else acc[t] += tmp[t];
           }
         }
@@ -460,7 +444,7 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_stream_kernel(StreamArgs a)
             m = ring_index[ring + r];
             if ((unsigned int)m >= (unsigned int)a.c_rows) continue;
           }
-          store_output4<MODE>(g, m, n, v);
+          store_output4<kModeBlock>(g, m, n, v);
         }
       }
     }
@@ -473,10 +457,10 @@ __global__ __launch_bounds__(kThreads) void fp8_gemm_stream_kernel(StreamArgs a)
 
 constexpr size_t part_bytes(int tmx) { return (size_t)kWaves * tmx * 256 * 4; }
 
-template <int TMX, int MODE>
+template <int TMX>
 int launch_stream_tmx(const StreamArgs& a, int grid, hipStream_t stream) {
   static PerDeviceFlags raised;
-  void (*const kern)(StreamArgs) = fp8_gemm_stream_kernel<TMX, MODE>;
+  void (*const kern)(StreamArgs) = fp8_gemm_stream_kernel<TMX>;
   const hipError_t e = raise_dynamic_lds_limit(raised, Cfg<TMX>::kLds, reinterpret_cast<const void*>(kern));
   if (e != hipSuccess) FG_FAIL(FG_ERR_LAUNCH, "hipFuncSetAttribute(%d bytes LDS): %s", Cfg<TMX>::kLds, hipGetErrorString(e));
   FG_LAUNCH(kern, dim3((uint32_t)grid), dim3(kThreads), Cfg<TMX>::kLds, stream, a);
@@ -498,8 +482,6 @@ int grouped_stream_rows(const GemmArgs& g, const GroupedGemm& gr) {
   return grouped_stream_pass_rows(g.M, g.N, g.KB, E, cu_count());
 }
 
-size_t stream_workspace_bytes() { return FG_WORKSPACE_COUNTER_BYTES + (size_t)512 * part_bytes(4); }
-
 int launch_grouped_stream(const GemmArgs& g, const GroupedGemm& gr, int rows, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   StreamArgs a = {};
   a.g = g;
@@ -518,9 +500,9 @@ int launch_grouped_stream(const GemmArgs& g, const GroupedGemm& gr, int rows, vo
     a.counters = reinterpret_cast<unsigned int*>(workspace);
     a.partials = reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + FG_WORKSPACE_COUNTER_BYTES);
   }
-  if (tmx == 1) return launch_stream_tmx<1, kModeBlock>(a, grid, stream);
-  if (tmx == 2) return launch_stream_tmx<2, kModeBlock>(a, grid, stream);
-  return launch_stream_tmx<4, kModeBlock>(a, grid, stream);
+  if (tmx == 1) return launch_stream_tmx<1>(a, grid, stream);
+  if (tmx == 2) return launch_stream_tmx<2>(a, grid, stream);
+  return launch_stream_tmx<4>(a, grid, stream);
 }
 
 }  // namespace fg
