@@ -106,7 +106,7 @@ def test_grouped_gemm_fp16():
     # the same sums as the bf16 call, rounded to the other type: never further from it than the two roundings allow
     bf = flag_gems.grouped_w8a8_block_fp8_matmul(*args).cpu().float()
     assert ((got.cpu().float() - bf).abs() <= bf.abs() * 2.0 ** -7 + 1e-6).all()
-    # few rows per segment (short tiles, tiles cut along K)
+    # few rows per segment (streaming kernel)
     ends2 = torch.tensor([5, 30, 30, 64], dtype=torch.int32)
     args2 = (xq[:64].to(DEV), wq.to(DEV), xs[:64].to(DEV), ws.to(DEV), ends2.to(DEV), [128, 128])
     got2 = flag_gems.grouped_w8a8_block_fp8_matmul(*args2, output_dtype=torch.float16)

@@ -104,3 +104,34 @@ def test_gather_scatter_weights_and_no_workspace(per):
         None, 0, _lib.current_stream_ptr(torch.device(DEV)))
     _lib.check(st, "fg_grouped_block_fp8_gemm")
     _close(c, want, mag)
+
+
+@pytest.mark.parametrize("per,K", [(2, 640), (14, 1024), (40, 896)])
+def test_scale_layouts_and_padded_rows(per, K):
+    """Column-major activation scales, and rows of every operand further apart than they are long: the bits of the plain call."""
+    E, N = 5, 392
+    counts = [per, 0, 2 * per, 1, per]
+    M = sum(counts)
+    x, w, xs, ws = _operands(M, N, K, E, seed=K)
+    ends = torch.tensor(counts).cumsum(0).int().to(DEV)
+    base = flag_gems.grouped_w8a8_block_fp8_matmul(x, w, xs, ws, ends, [128, 128])
+    assert torch.equal(flag_gems.grouped_w8a8_block_fp8_matmul(x, w, xs.t().contiguous().t(), ws, ends, [128, 128]), base)
+    lda, ldb, ldc, rows = K + 48, K + 16, N + 24, N + 3
+    xp = torch.full((M, lda), 0x7F, dtype=torch.uint8, device=DEV)  # NaN codes between the rows
+    xp[:, :K] = x.view(torch.uint8)
+    wp = torch.full((E, rows, ldb), 0x7F, dtype=torch.uint8, device=DEV)
+    wp[:, :N, :K] = w.view(torch.uint8)
+    xsp = torch.full((M, xs.shape[1] + 5), float("nan"), device=DEV)
+    xsp[:, :xs.shape[1]] = xs
+    wsp = torch.full((E, ws.shape[1] + 1, ws.shape[2] + 2), float("nan"), device=DEV)
+    wsp[:, :ws.shape[1], :ws.shape[2]] = ws
+    c = torch.zeros(M, ldc, dtype=torch.bfloat16, device=DEV)
+    lib = _lib.load()
+    size = lib.fg_grouped_block_fp8_gemm_workspace_bytes(M, N, K)
+    work = torch.zeros(size, dtype=torch.uint8, device=DEV)
+    st = lib.fg_grouped_block_fp8_gemm(
+        xp.data_ptr(), lda, wp.data_ptr(), ldb, rows * ldb, xsp.data_ptr(), xsp.stride(0), 1, wsp.data_ptr(), wsp.stride(1), 1, wsp.stride(0),
+        ends.data_ptr(), E, None, 1, M, 0, None, c.data_ptr(), ldc, _lib.DTYPE_CODE[torch.bfloat16], M, N, K, 128, 128,
+        work.data_ptr(), size, _lib.current_stream_ptr(torch.device(DEV)))
+    _lib.check(st, "fg_grouped_block_fp8_gemm")
+    assert torch.equal(c[:, :N], base) and not c[:, N:].any()
