@@ -668,15 +668,15 @@ int launch_tile_split(GemmArgs a, const TileSplitPlan& plan, void* workspace, hi
   return FG_OK;
 }
 
-// M >= 65 with at most one 128 x 128 tile per compute unit: the tile kernel with four LDS stages, one block
-// per compute unit, K split over blocks while blocks are fewer than compute units.  With two stages a block that
+// M >= 65 with at most one tile per compute unit: the tile kernel with four LDS stages on 128 x 128 tiles (three on 256 x 128
+// tiles where tall_tiles_pay says so; the rest of this comment is about the former), one block per compute unit, K split over blocks while blocks are fewer than compute units.  With two stages a block that
 // has a compute unit to itself pays a whole load latency per K-block.  The tile count decides, not M: tall
 // problems against narrow weights (M = 2048, N = 512, K = 7168: 128 tiles) took 73 us in the persistent kernel, which
 // has a quarter of the tiles and shares them along K, and take 22 us here; with more tiles than compute units a
 // second round of this kernel loses to the persistent kernel (M = 1024, N = 4608, K = 7168, 288 tiles: 62 -> 79 us).
 struct PipePlan {
   bool use;
-  bool tall;  // 256 x 128 tiles, three stages
+  bool tall;  // 256 x 128 tiles, three stages, never split along K
   int splits, kb_per_split;
   size_t workspace_bytes;
 };
@@ -945,12 +945,13 @@ int launch_gemm(const GemmArgs& a, void* workspace, size_t workspace_bytes, hipS
   }
   {
     const int64_t tiles128 = ceil_div(a.M, 128) * ceil_div(a.N, 128);
-    // 257..512 tiles of 128 x 128 with K up to 4096: at most the 512 workgroups that are
-    // resident at a time, two on each compute unit (560 tiles: M = 1280, N = 7168, K = 2304 went from 36 to 51 us); the persistent kernel has a quarter of the tiles and spends its
-    // time filling and draining.  Measured: M = 256, N = 24576, K = 1536: 27.7 -> 23.4 us; M = 768, N = 7168, K = 2304:
-    // 34.8 -> 28.9; N = 6144, K = 4096: 50.0 -> 43.4; M = 1024, N = 7168, K = 2304: 35.3 -> 29.6.
-    // The tile count decides, whatever M: M = 2048, N = 3072, K = 2048: 34.0 -> 24.8 us; M = 3072, N = K = 2048: 34.0 -> 24.2;
-    // M = 2048, N = K = 4096: 51.0 -> 45.2.
+    // 257..512 tiles of 128 x 128 with K up to 4096 that tall tiles did not take: at most the 512 workgroups that are
+    // resident at a time, two on each compute unit (560 tiles: M = 1280, N = 7168, K = 2304 went from 36 to 51 us); the persistent
+    // kernel has a quarter of the tiles and spends its time filling and draining.  Mostly row and column scales, and block
+    // scales with few K-blocks or few more tiles than units.  Persistent -> here, block scales, before there were tall tiles
+    // (which most of these take now, see tall_tiles_pay): M = 256, N = 24576, K = 1536: 27.7 -> 23.4 us; M = 768, N = 7168, K = 2304:
+    // 34.8 -> 28.9; N = 6144, K = 4096: 50.0 -> 43.4; M = 1024, N = 7168, K = 2304: 35.3 -> 29.6.  The tile count decides, whatever M: M = 2048,
+    // N = 3072, K = 2048: 34.0 -> 24.8 us; M = 3072, N = K = 2048: 34.0 -> 24.2; M = 2048, N = K = 4096: 51.0 -> 45.2.
     // With longer K the persistent kernel, which shares tiles between compute units through the workspace, is ahead: the rule
     // once reached to K = 8192 for up to 448 tiles, and without that M = 256, N = 20480, K = 8192 goes from 100 to 72 us; M = 512,
     // N = 10240: 92 -> 65; M = 384, N = 14336: 91 -> 78; M = 768, N = 7168: 85 -> 65; M = 512, N = 9216, K = 6144: 73 -> 55; M = 256,

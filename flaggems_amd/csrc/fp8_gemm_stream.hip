@@ -4,7 +4,7 @@
 // Bound: HBM (the weights are read once, 32 .. 128 flops a byte).  Measured, weight bytes of the groups that have rows
 // over the launch's time: 512 groups of [2048, 4096], one or two rows each, 5.9 TB/s (the persistent kernel's 64-row tiles:
 // 1.2); 8 groups of [28672, 4096], 1 .. 8 rows each, 5.4 - 5.7 TB/s (4.4 - 4.6), 48 rows each 4.8 (4.0); 8 of
-// [4096, 14336] 5.2 - 5.6 (3.3 - 4.2).  A copy of 2 GB moves 4.9 TB/s on the same part.  What the design is about is keeping every compute
+// [4096, 14336] 5.2 - 5.6 (3.3 - 4.2).  A copy of 1 GiB moves 4.9 - 5.1 TB/s.  What the design is about is keeping every compute
 // unit's queue of weight loads full from the first to the last byte of the launch, whatever the table of groups says.
 //
 //  * A step is 128 weight rows x 256 bytes of K (two K-blocks) against up to 16 TMX activation rows.  An item is one
