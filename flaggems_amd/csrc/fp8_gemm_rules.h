@@ -24,6 +24,9 @@ namespace fg {
 //     N = 7168, K = 2304: 7 % and more), but where the weights set the time: up to two tile rows and enough K (M = 136, N = 28672, K = 4096:
 //     45.0 -> 40.4; M = 479, N = 11648, K = 4096: 43.0 -> 38.5; but M = 200, N = 16832, K = 2176, 264 tiles: 24.7 -> 26.7).
 //   * four K-blocks (M = 256, N = 20480, K = 512: 11.9 -> 12.3), and more than 64, which nobody measured.
+// The figures are for 16-bit results.  fp32 results with block scales gain as much or more (median 0.6 beyond 32 K-blocks); fp32 and
+// fp8 results with row and column scales have the 128-row kernel as their alternative there too: median 0.85 - 0.96 up to four tile
+// rows, 0.92 - 1.03 with more (1.08 at worst).
 // Split along K such tiles lose to 128-row ones (M = 256: N = K = 8192 in four: 36.5 -> 41.4): twice the partial sums.
 inline bool tall_tiles_pay(bool block_scales, int64_t M, int64_t N, int64_t k_blocks, int64_t cus) {
   if (M <= 128 || k_blocks < 8 || k_blocks > 64) return false;
