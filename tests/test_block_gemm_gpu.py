@@ -538,3 +538,23 @@ def test_parts_that_share_rows_agree_bit_for_bit(rows, stride, parts, N, K, dtyp
         torch.testing.assert_close(c[z].cpu().float(), want[z * stride:z * stride + rows], **tol)
         if z + 1 < parts:
             assert torch.equal(c[z][stride:].view(torch.int8), c[z + 1][:shared].view(torch.int8))
+
+
+@pytest.mark.parametrize("M", [129, 130, 134, 145, 164, 193, 209, 257, 270, 300, 511])
+def test_many_parts_write_no_row_past_the_last(M):
+    """Sixteen and thirty-two parts whose rows run out before the parts do: nothing past the last row is written, and every row
+    is right."""
+    from flaggems_amd import _lib
+    lib = _lib.load()
+    N, K = 832, 1152
+    xq, wq, xs, ws = (t.to(DEV) for t in _quantized_inputs(M, N, K, seed=M))
+    kb = K // 128
+    c = torch.full((M + 64, N), 7.0, dtype=torch.bfloat16, device=DEV)
+    need = lib.fg_block_fp8_gemm_workspace_bytes(M, N, K)
+    wsp = _lib.workspace(torch.device(DEV), max(need, 1))
+    rc = lib.fg_block_fp8_gemm(xq.data_ptr(), K, wq.data_ptr(), K, xs.data_ptr(), kb, 1, ws.data_ptr(), kb, 1, c.data_ptr(), N, _lib.FG_BF16,
+                               M, N, K, 128, 128, wsp.data_ptr(), wsp.numel(), _lib.current_stream_ptr(torch.device(DEV)))
+    _lib.check(rc, "fg_block_fp8_gemm")
+    assert (c[M:] == 7.0).all()
+    want = O.block_fp8_matmul_dequant_ref(xq.cpu(), wq.cpu(), xs.cpu(), ws.cpu(), [128, 128], torch.float32, torch.float64)
+    torch.testing.assert_close(c[:M].cpu().float(), want, rtol=1e-2, atol=1e-2)

@@ -14,6 +14,11 @@ extern "C" int tall(int block, long long M, long long N, long long kb, long long
 extern "C" int stream_rows(long long M, long long N, long long kb, long long groups, long long cus) {
   return fg::grouped_stream_pass_rows(M, N, kb, groups, cus);
 }
+extern "C" int parts(long long M, long long N, long long K, long long* rows, long long* back) {
+  const fg::DecodeParts d = fg::decode_parts(M, N, K);
+  *rows = d.rows, *back = d.back;
+  return (int)d.parts;
+}
 extern "C" int copy_rows(long long M, long long N, long long K, long long groups, long long cus) { return fg::gather_copy_pays(M, N, K, groups, cus); }
 """ % HEADER
 
@@ -31,7 +36,23 @@ def rules(tmp_path_factory):
     so = ctypes.CDLL(lib)
     so.tall.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
     so.stream_rows.argtypes = so.copy_rows.argtypes = [ctypes.c_longlong] * 5
+    so.parts.argtypes = [ctypes.c_longlong] * 3 + [ctypes.POINTER(ctypes.c_longlong)] * 2
     return so
+
+
+def test_parts_of_the_rows_stay_inside_the_matrix(rules):
+    """Every part begins a part's rows after the one before and ends inside the matrix; only the last one is moved back."""
+    rows, back = ctypes.c_longlong(), ctypes.c_longlong()
+    taken = 0
+    for N, K in ((512, 512), (832, 1152), (576, 7168), (1024, 2048), (1536, 7168), (4096, 512), (6144, 8192), (8192, 1024)):
+        for M in range(1, 600):
+            n = rules.parts(M, N, K, ctypes.byref(rows), ctypes.byref(back))
+            if n == 0:
+                continue
+            taken += 1
+            assert 1 <= rows.value <= 16 and 0 <= back.value < rows.value
+            assert (n - 1) * rows.value <= M and n * rows.value - back.value == M
+    assert taken > 1000
 
 
 # block scales?, M, N, K, us on the 256 x 128 tiles, us on the kernel that serves the shape otherwise
