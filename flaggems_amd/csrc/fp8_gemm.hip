@@ -819,6 +819,14 @@ int launch_gemm(const GemmArgs& a, void* workspace, size_t workspace_bytes, hipS
   const bool direct = (a.K > 0) && (a.K % 128 == 0) && (a.ldx % 16 == 0) && (a.ldw % 16 == 0) &&
                       (a.ldx < (1 << 23)) && (a.ldw < (1 << 23)) &&
                       ((uintptr_t)a.X % 16 == 0) && ((uintptr_t)a.W % 16 == 0);
+  // up to 128 rows: both operands through LDS, the weights read once (where that is the faster one: plan_skinny); the kernels below take
+  // the rest, and calls without the workspace that a split K needs
+  if (direct && a.batch <= 1) {
+    const SkinnyPlan sk = plan_skinny(a.M, a.N, a.K, MODE == kModeBlock);
+    if (sk.use && (MODE != kModeBlock || skinny_takes_scales(a, sk)) &&
+        (sk.splits == 1 || (workspace != nullptr && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= sk.workspace_bytes)))
+      return launch_skinny(a, MODE, sk, workspace, stream);
+  }
   // 17..128 rows against narrow or small weights: parts of up to 16 rows on the decode kernels in one launch (the entries of a
   // batch that shares the weights).  With 17 rows or more a decode block fetches 32 activation rows per 16-32 weight rows
   // through registers; with up to 16 the activations of its K range lie in LDS.  Every part reads the weights again, so
@@ -990,6 +998,10 @@ extern "C" size_t fg_block_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_
       const size_t both = FG_WORKSPACE_COUNTER_BYTES + (size_t)parts * (mh.workspace_bytes - FG_WORKSPACE_COUNTER_BYTES);
       if (both > need) need = both;
     }
+  }
+  for (const bool block_scales : {false, true}) {
+    const fg::SkinnyPlan sk = fg::plan_skinny(M, N, K, block_scales);
+    if (sk.use && sk.workspace_bytes > need) need = sk.workspace_bytes;
   }
   const size_t pp = fg::pingpong_workspace_bytes(M, N, K);
   return pp > need ? pp : need;

@@ -255,6 +255,18 @@ MidMPlan plan_mid_m(int64_t M, int64_t N, int64_t K, int64_t entries = 1);
 int launch_mid_m(const GemmArgs& a, int mode, const MidMPlan& plan, void* workspace, size_t workspace_bytes,
                  hipStream_t stream);
 
+// Up to 128 rows, fp8_gemm_skinny.hip: both operands through LDS in deep stages, the weights read once.
+struct SkinnyPlan {
+  bool use;
+  int cfg;                       // tile and ring (kShapes)
+  int tiles_n;                   // tiles along N
+  int splits, stages_per_split;  // blocks along K, and the 256-byte stages of each
+  size_t workspace_bytes;
+};
+SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales);
+bool skinny_takes_scales(const GemmArgs& a, const SkinnyPlan& plan);
+int launch_skinny(const GemmArgs& a, int mode, const SkinnyPlan& plan, void* workspace, hipStream_t stream);
+
 // Persistent 256x256 kernel, fp8_gemm_pingpong.hip: bf16 output with 16-byte aligned rows, M > 128 (or M > 64 when
 // the workspace lets it share tiles along K);
 // the caller has checked that the operands qualify for direct global->LDS loads.
