@@ -178,6 +178,31 @@ def fast():
     return _fast
 
 
+_host = None
+
+
+def host():
+    """The native host side of the block GEMM and the group quantizer (csrc/hostcalls.cpp, built next to the library by
+    flaggems_amd/build.py): its functions return None for whatever is not the plain case, which the Python code then serves."""
+    global _host
+    if _host is None:
+        import importlib.util
+
+        from .build import hostcalls_path
+
+        path = hostcalls_path()
+        if not os.path.exists(path):
+            raise ImportError(f"{path} is missing: build it with `python -m flaggems_amd.build`")
+        spec = importlib.util.spec_from_file_location("_fg_hostcalls", path)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        if _raw_stream is not None:  # (without it every call is left to the Python code)
+            mod.connect(address("fg_block_fp8_gemm"), address("fg_block_fp8_gemm_pow2_scales"), address("fg_block_fp8_gemm_workspace_bytes"),
+                        address("fg_group_quant_fp8"), workspace, check, _raw_stream)
+        _host = mod
+    return _host
+
+
 def address(name: str) -> int:
     """Address of an exported C function, for the calls that go through `fast()`."""
     a = _addresses.get(name)

@@ -170,6 +170,12 @@ def per_token_group_quant_fp8(
     """
     logger.debug("GEMS PER TOKEN GROUP QUANT FP8")
     fp8_dtype = SUPPORTED_FP8_DTYPE if dtype is None else dtype
+    if scale_rule is None and fp8_dtype is torch.float8_e4m3fn and x.is_cuda and x.dtype in _IN_DTYPES:  # a matrix: one native call
+        rule_code, floor = _default_rule_and_floor(eps, x.dtype)
+        pair = _lib.host().group_quant(x, group_size, column_major_scales, floor, rule_code, _lib.FG_QUOT_DIV,
+                                       _lib.FG_POW2_LOG2 if scale_ue8m0 else _lib.FG_POW2_NONE)
+        if pair is not None:
+            return pair
     assert x.shape[-1] % group_size == 0, (
         f"the last dimension of `x` {x.shape[-1]} must be divisible "
         f"by `group_size` {group_size}"

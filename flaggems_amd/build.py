@@ -82,6 +82,38 @@ def build_fastcall(verbose: bool = True) -> str:
     return out
 
 
+HOSTCALLS_SRC = os.path.join(CSRC, "hostcalls.cpp")
+
+
+def hostcalls_path() -> str:
+    import sysconfig
+
+    return os.path.join(HERE, "_fg_hostcalls" + (sysconfig.get_config_var("EXT_SUFFIX") or ".so"))
+
+
+def build_hostcalls(verbose: bool = True) -> str:
+    """Compile the native host side of the decode-critical calls (csrc/hostcalls.cpp) against torch's headers.  It links
+    torch's libraries, which the process has loaded by the time it is imported, and nothing of libflaggems_amd.so."""
+    import sysconfig
+
+    import torch
+
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("no host C++ compiler (g++ / c++) for csrc/hostcalls.cpp")
+    root = os.path.dirname(torch.__file__)
+    out = hostcalls_path()
+    tmp = out + ".tmp"
+    _run([cxx, "-std=c++17", "-O2", "-shared", "-fPIC", "-Wall", "-D_GLIBCXX_USE_CXX11_ABI=%d" % torch._C._GLIBCXX_USE_CXX11_ABI,
+          "-I" + sysconfig.get_paths()["include"], "-isystem", os.path.join(root, "include"),
+          "-isystem", os.path.join(root, "include", "torch", "csrc", "api", "include"), HOSTCALLS_SRC, "-o", tmp,
+          "-L" + os.path.join(root, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10"])
+    os.replace(tmp, out)
+    if verbose:
+        print("[flaggems_amd.build] built", out, flush=True)
+    return out
+
+
 def build(verbose: bool = True, jobs: int = 4) -> str:
     """Compile every HIP source for gfx950 and link the shared library.  Always recompiles."""
     hipcc = _hipcc()
@@ -105,6 +137,7 @@ def build(verbose: bool = True, jobs: int = 4) -> str:
     if verbose:
         print("[flaggems_amd.build] linked", LIB_PATH, flush=True)
     build_fastcall(verbose)
+    build_hostcalls(verbose)
     return LIB_PATH
 
 

@@ -87,6 +87,10 @@ def w8a8_block_fp8_matmul(
     logger.debug("GEMS W8A8_BLOCK_FP8_MATMUL")
     assert len(block_size) == 2
     block_n, block_k = block_size[0], block_size[1]
+    if A.is_cuda:  # contiguous matrices and 128 x 128 scale blocks, as a model's linears have them: one native call
+        C = _lib.host().block_matmul(A, B, As, Bs, block_n, block_k, output_dtype, scales_are_powers_of_two)
+        if C is not None:
+            return C
 
     assert A.shape[-1] == B.shape[-1]
     assert A.shape[:-1] == As.shape[:-1] and A.is_contiguous()
