@@ -28,11 +28,12 @@ namespace {
 // Map the hardware block id to a tile so that (a) the blocks one XCD receives (ids congruent mod 8)
 // form a contiguous run of tiles and (b) a run walks GROUP_M tile rows before moving along N, which
 // keeps the 32 tiles resident on an XCD inside a compact patch that shares operand panels in its L2.
-__device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n, int& tm, int& tn) {
+// `in_order`: the ids are those of one XCD already.
+__device__ __forceinline__ void tile_of_block(int bid, int tiles_m, int tiles_n, bool in_order, int& tm, int& tn) {
   const int total = tiles_m * tiles_n;
   const int xcd = bid & 7, local = bid >> 3;
   const int base = total >> 3, rem = total & 7;
-  const int sid = xcd * base + (xcd < rem ? xcd : rem) + local;
+  const int sid = in_order ? bid : xcd * base + (xcd < rem ? xcd : rem) + local;
   constexpr int GROUP_M = 4;
   const int per_group = GROUP_M * tiles_n;
   const int g = sid / per_group;
@@ -213,12 +214,27 @@ struct TileCfg {
 // the one that arrives last adds the sums of all splits in split order -- the same order whoever comes last --
 // and runs the epilogue.  For problems with few tiles, which would leave most of the GPU idle while every
 // K-block of a tile costs a full load latency.
-template <int BM, int BN, int WM, int WN, int MODE, bool DIRECT, bool SPLIT = false, int NST = 2>
+// BATCH: a.batch equal problems in one launch (blockIdx.y).
+template <int BM, int BN, int WM, int WN, int MODE, bool DIRECT, bool SPLIT = false, int NST = 2, bool BATCH = false>
 __global__ __launch_bounds__(WM* WN * 64) void fp8_gemm_kernel(GemmArgs a) {
   using Cfg = TileCfg<BM, BN, WM, WN, NST>;
   static_assert(NST == 2 || (DIRECT && NST >= 3 && NST <= 5), "deep pipeline: direct loads, 3..5 stages");
-  if (a.batch > 1) {  // uniform: this workgroup's entry of the batch
-    const int64_t z = blockIdx.y;
+  int block = (int)blockIdx.x;
+  const bool own_entries = BATCH && (a.batch >= 8 || (a.batch >= 4 && a.splits <= 1));
+  if constexpr (BATCH) {  // uniform: this workgroup's entry of the batch
+    // Every XCD works through entries of its own (ids congruent mod 8 share one): its L2 then holds the panels of one entry's tiles
+    // instead of a slice of every entry's.  8 entries of [500, 8192] x [1024, 8192]: 12 distinct panels of a K-block for the 32 tiles of
+    // an XCD instead of 40, 58.4 -> 55.1 us; 1500 rows of 8 x [512, 4096]: 51.1 -> 43.6.  Not with few entries: two (1000 rows of
+    // [512, 4096]) 17.3 -> 21.0, four with K split (129 rows of [1024, 8192]) 22.7 -> 23.7.
+    int64_t z = blockIdx.y;
+    if (own_entries) {
+      const int per_entry = (int)gridDim.x, total = per_entry * a.batch;
+      const int id = (int)(blockIdx.y * gridDim.x + blockIdx.x), share = total >> 3, rem = total & 7, xcd = id & 7;
+      const int at = xcd * share + (xcd < rem ? xcd : rem) + (id >> 3);
+      const int entry = at / per_entry;
+      block = at - entry * per_entry;
+      z = entry;
+    }
     a.X += z * a.x_batch_bytes;
     a.W += z * a.w_batch_bytes;
     a.C = reinterpret_cast<uint8_t*>(a.C) + z * a.c_batch_bytes;
@@ -241,16 +257,16 @@ __global__ __launch_bounds__(WM* WN * 64) void fp8_gemm_kernel(GemmArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wave_m = wave % WM, wave_n = wave / WM;
 
-  int tile_id = (int)blockIdx.x, split = 0;
+  int tile_id = block, split = 0;
   if (SPLIT) {
     const int n_tiles = a.tiles_m * a.tiles_n;
-    split = (int)blockIdx.x / n_tiles;
-    tile_id = (int)blockIdx.x - split * n_tiles;
+    split = block / n_tiles;
+    tile_id = block - split * n_tiles;
   }
   const int kb_begin = SPLIT ? split * a.kb_per_split : 0;
   const int kb_end = SPLIT ? (kb_begin + a.kb_per_split < a.KB ? kb_begin + a.kb_per_split : a.KB) : a.KB;
   int tile_m, tile_n;
-  tile_of_block(tile_id, a.tiles_m, a.tiles_n, tile_m, tile_n);
+  tile_of_block(tile_id, a.tiles_m, a.tiles_n, own_entries, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   const int wm0 = wave_m * Cfg::kWaveM, wn0 = wave_n * Cfg::kWaveN;
   const int l16 = lane & 15, lg = lane >> 4;
@@ -591,12 +607,12 @@ __global__ __launch_bounds__(WM* WN * 64) void fp8_gemm_kernel(GemmArgs a) {
   }
 }
 
-template <int BM, int BN, int WM, int WN, int MODE, bool DIRECT>
+template <int BM, int BN, int WM, int WN, int MODE, bool DIRECT, bool BATCH = false>
 int launch_cfg(GemmArgs a, hipStream_t stream) {
   using Cfg = TileCfg<BM, BN, WM, WN>;
   a.tiles_m = (int)ceil_div(a.M, BM);
   a.tiles_n = (int)ceil_div(a.N, BN);
-  auto kern = fp8_gemm_kernel<BM, BN, WM, WN, MODE, DIRECT>;
+  auto kern = fp8_gemm_kernel<BM, BN, WM, WN, MODE, DIRECT, false, 2, BATCH>;
   static PerDeviceFlags lds_limit_raised = {};  // per instantiation
   {
     const hipError_t e = raise_dynamic_lds_limit(lds_limit_raised, Cfg::kLdsBytes, reinterpret_cast<const void*>(kern));
@@ -604,7 +620,7 @@ int launch_cfg(GemmArgs a, hipStream_t stream) {
   }
   const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n;
   if (blocks > 0x7FFFFFFF) FG_FAIL(FG_ERR_UNSUPPORTED, "fp8 gemm: too many tiles");
-  if (a.batch > 65535) FG_FAIL(FG_ERR_UNSUPPORTED, "fp8 gemm: more than 65535 batch entries in one launch");
+  if (a.batch > 65535 || (a.batch > 1 && !BATCH)) FG_FAIL(FG_ERR_UNSUPPORTED, "fp8 gemm: a batch of %d in one launch", a.batch);
   FG_LAUNCH(kern, dim3((uint32_t)blocks, (uint32_t)(a.batch > 1 ? a.batch : 1)), dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, a);
   FG_CHECK_LAUNCH("fp8_gemm_kernel");
   return FG_OK;
@@ -764,13 +780,16 @@ int launch_pipe_tile(GemmArgs a, const PipePlan& plan, void* workspace, hipStrea
   a.split_partials = workspace && plan.splits > 1 ? reinterpret_cast<float*>(reinterpret_cast<uint8_t*>(workspace) + FG_WORKSPACE_COUNTER_BYTES) : nullptr;
   a.split_partials_per_entry = (int64_t)a.tiles_m * a.tiles_n * a.splits * BM * kSplitTile;
   auto kern = fp8_gemm_kernel<BM, kSplitTile, kSplitWM, 2, MODE, true, true, NST>;
+  constexpr bool kBatches = MODE == kModeBlock && NST == kPipeStages;
+  auto batched = fp8_gemm_kernel<BM, kSplitTile, kSplitWM, 2, MODE, true, true, NST, kBatches>;
+  if (a.batch > 1 && !kBatches) FG_FAIL(FG_ERR_UNSUPPORTED, "fp8 gemm (deep pipeline): a batch of %d", a.batch);
   static PerDeviceFlags lds_limit_raised = {};
   {
-    const hipError_t e = raise_dynamic_lds_limit(lds_limit_raised, Cfg::kLdsBytes, reinterpret_cast<const void*>(kern));
+    const hipError_t e = raise_dynamic_lds_limit(lds_limit_raised, Cfg::kLdsBytes, reinterpret_cast<const void*>(kern), reinterpret_cast<const void*>(batched));
     if (e != hipSuccess) FG_FAIL(FG_ERR_LAUNCH, "hipFuncSetAttribute(%d bytes LDS): %s", Cfg::kLdsBytes, hipGetErrorString(e));
   }
   const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n * a.splits;
-  FG_LAUNCH(kern, dim3((uint32_t)blocks, (uint32_t)(a.batch > 1 ? a.batch : 1)), dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, a);
+  FG_LAUNCH(a.batch > 1 ? batched : kern, dim3((uint32_t)blocks, (uint32_t)(a.batch > 1 ? a.batch : 1)), dim3(Cfg::kThreads), Cfg::kLdsBytes, stream, a);
   FG_CHECK_LAUNCH("fp8_gemm_kernel (deep pipeline)");
   return FG_OK;
 }
@@ -1218,8 +1237,8 @@ extern "C" int fg_batched_block_fp8_gemm(const void* A, int64_t lda, int64_t a_b
       }
       // 256 x 256 tiles once the batch has one for every compute unit (measured, h = 8, r = 4096, d = 1024, 128-row against
       // 256-row tiles: b = 1024: 54 against 74 us; b = 2048: 101 against 84; b = 4096: 208 against 160 us = 1.72 PFLOP/s)
-      if (batch * big_tiles >= 256) return launch_cfg<256, 256, 4, 2, kModeBlock, true>(a, (hipStream_t)stream);
-      return launch_cfg<128, 128, 2, 2, kModeBlock, true>(a, (hipStream_t)stream);
+      if (batch * big_tiles >= 256) return launch_cfg<256, 256, 4, 2, kModeBlock, true, true>(a, (hipStream_t)stream);
+      return launch_cfg<128, 128, 2, 2, kModeBlock, true, true>(a, (hipStream_t)stream);
     }
   }
   // One launch per matrix, in batch order on the caller's stream: each is the plain GEMM of its operands (same
