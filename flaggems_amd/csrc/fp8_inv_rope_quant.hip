@@ -11,8 +11,8 @@
 //
 // A wavefront takes one head of one token per step: 64 lanes x 8 values cover a head of 512 (longer heads take further
 // passes), a rotated pair lies inside a lane, a 128-value group is 16 adjacent lanes (DPP maximum), and the eight lanes
-// that hold the rope tail fetch their cos/sin once per token.  A wavefront walks HPW consecutive heads of a token with
-// all loads issued first, then the next of its tokens.  HBM bound: 3 bytes per bf16 value.
+// that hold the rope tail fetch their cos/sin once per token.  A wavefront takes HPW consecutive heads of one token, all
+// loads issued first.  HBM bound: 3 bytes per bf16 value.
 
 #include "fp8_quant_device.h"
 
@@ -20,7 +20,7 @@ namespace fg {
 namespace {
 
 constexpr int kRopeThreads = 256;
-constexpr int kRopeWaves = kRopeThreads / 64;
+constexpr int kRopeTokens = kRopeThreads / 64;  // tokens of a workgroup, one per wavefront
 
 struct InvRopeArgs {
   const void* o;
@@ -48,11 +48,14 @@ __device__ __forceinline__ void rotate_back(float (&xv)[8], const float (&c)[4],
 }
 
 // Scales of one token are chunks * heads words scattered over as many columns (tokens have unit stride): a workgroup
-// therefore takes kRopeTokens (16, or 4 in small launches) consecutive tokens of the same HPW heads, collects their scales in LDS and writes every
-// column's words of those tokens as one run.
+// therefore takes kRopeTokens consecutive tokens of the same HPW heads, collects their scales in LDS and writes every
+// column's words of those tokens as one run.  (Four tokens, 16-byte runs: with sixteen, a wavefront walked four tokens one after the other,
+// waiting for the position, the angles and the values of each, and the launch had a quarter of the workgroups.  bf16, heads x 512:
+// 256 x 128 19.5 -> 16.5 us, 500 x 128 29.0 -> 25.8, 1024 x 128 49.4 -> 46.0, 4096 x 128 168 -> 170; fetching the next token's values under the
+// current one's arithmetic instead cost more registers than it saved: 500 x 128 29.0 -> 36.5.)
 constexpr int kRopeLdsChunks = 16;  // groups per head that the LDS rows hold; longer heads store their scales directly
 
-template <int XDT, int LPG, int HPW, int kRopeTokens, bool PACKED>
+template <int XDT, int LPG, int HPW, bool PACKED>
 __global__ __launch_bounds__(kRopeThreads) void inv_rope_quant_kernel(InvRopeArgs a, int padded_tokens, int head_blocks) {
   // the rules are fixed for this producer: as constants they leave no rule switch in the loop
   a.qa.scale_rule = FG_SCALE_MUL_INV;
@@ -74,9 +77,8 @@ __global__ __launch_bounds__(kRopeThreads) void inv_rope_quant_kernel(InvRopeArg
   for (int i = threadIdx.x; i < HPW * kRopeLdsChunks * kRopeTokens; i += kRopeThreads) (&rows[0][0])[i] = 0u;
   __syncthreads();
 
-  for (int tl = wave; tl < kRopeTokens; tl += kRopeWaves) {
-    const int64_t t = t0 + tl;
-    if (t >= a.tokens) break;  // uniform over the wavefront
+  const int tl = wave;
+  if (const int64_t t = t0 + tl; t < a.tokens) {  // uniform over the wavefront
     int64_t pos = a.pos_bytes == 8 ? reinterpret_cast<const int64_t*>(a.positions)[t]
                                    : (int64_t)reinterpret_cast<const int32_t*>(a.positions)[t];
     // the reference reads whatever lies at an out-of-range position; here the access stays inside the cache
@@ -177,16 +179,18 @@ __global__ __launch_bounds__(kRopeThreads) void inv_rope_quant_kernel(InvRopeArg
 
 template <int XDT, int LPG>
 int launch_inv_rope(const InvRopeArgs& a, int64_t padded_tokens, hipStream_t stream) {
-  // 16 tokens and four heads per workgroup once that leaves workgroups enough to fill the GPU; else 4 tokens, one head
-  const bool wide = ceil_div(padded_tokens, (int64_t)16) * (a.heads / 4) >= 1024 && a.heads % 4 == 0;
-  const int64_t head_blocks = wide ? a.heads / 4 : a.heads;
-  const int64_t blocks = ceil_div(padded_tokens, (int64_t)(wide ? 16 : 4)) * head_blocks;
+  // Heads a wavefront takes, us for one / two / four (tokens x heads, bf16): 16 x 128 4.0 / 4.3 / 5.5; 61 x 64 4.9 / 5.2 / 6.1; 61 x 128 6.9 / 6.6 / 7.2;
+  // 150 x 64 7.8 / 7.4 / 8.2; 150 x 128 11.9 / 10.9 / 10.8; 500 x 128 - / 27.5 / 25.8; 2048 x 128 127 / 99.6 / 89.2.  fp32, whose values take twice the
+  // registers: 61 x 128 7.0 / 7.4 / 8.3; 150 x 128 13.2 / 12.7 / 13.3; 2048 x 128 135 / 129 / 132.
+  const int64_t pieces = ceil_div(padded_tokens, (int64_t)kRopeTokens) * a.heads;
+  const int hpw = XDT != FG_F32 && pieces >= 4864 && a.heads % 4 == 0 ? 4 : pieces >= (XDT == FG_F32 ? 2400 : 2048) && a.heads % 2 == 0 ? 2 : 1;
+  const int64_t head_blocks = a.heads / hpw, blocks = pieces / hpw;
   if (blocks > 0x7FFFFFFF) FG_FAIL(FG_ERR_UNSUPPORTED, "fg_inv_rope_group_quant_fp8: too many workgroups");
-  const dim3 grid((uint32_t)blocks);
-  if (wide && a.packed) FG_LAUNCH((inv_rope_quant_kernel<XDT, LPG, 4, 16, true>), grid, dim3(kRopeThreads), 0, stream, a, (int)padded_tokens, (int)head_blocks);
-  else if (wide) FG_LAUNCH((inv_rope_quant_kernel<XDT, LPG, 4, 16, false>), grid, dim3(kRopeThreads), 0, stream, a, (int)padded_tokens, (int)head_blocks);
-  else if (a.packed) FG_LAUNCH((inv_rope_quant_kernel<XDT, LPG, 1, 4, true>), grid, dim3(kRopeThreads), 0, stream, a, (int)padded_tokens, (int)head_blocks);
-  else FG_LAUNCH((inv_rope_quant_kernel<XDT, LPG, 1, 4, false>), grid, dim3(kRopeThreads), 0, stream, a, (int)padded_tokens, (int)head_blocks);
+  const dim3 grid((uint32_t)blocks), block(kRopeThreads);
+  auto go = [&](auto plain, auto packed) { FG_LAUNCH(a.packed ? packed : plain, grid, block, 0, stream, a, (int)padded_tokens, (int)head_blocks); };
+  if (hpw == 4) go(inv_rope_quant_kernel<XDT, LPG, XDT == FG_F32 ? 2 : 4, false>, inv_rope_quant_kernel<XDT, LPG, XDT == FG_F32 ? 2 : 4, true>);
+  else if (hpw == 2) go(inv_rope_quant_kernel<XDT, LPG, 2, false>, inv_rope_quant_kernel<XDT, LPG, 2, true>);
+  else go(inv_rope_quant_kernel<XDT, LPG, 1, false>, inv_rope_quant_kernel<XDT, LPG, 1, true>);
   return FG_OK;
 }
 

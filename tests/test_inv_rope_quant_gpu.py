@@ -268,3 +268,13 @@ def test_benchmark_size_by_sample_and_property():
     assert_scales_equal(sc[pick.to(DEV)], want_s, "sample")
     top = out.view(torch.uint8).reshape(tokens, groups, -1, GROUP).bitwise_and(0x7F).amax(dim=-1)
     assert bool((top == 0x7E).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tma", [False, True])
+@pytest.mark.parametrize("num_tokens,num_heads,n_groups", [(61, 128, 8), (149, 128, 8), (153, 128, 8), (1217, 16, 2), (2430, 6, 2)])
+def test_heads_a_wavefront_takes(num_tokens, num_heads, n_groups, tma, dtype):
+    """Either side of the lines where a wavefront goes over from one head to two and to four, a token count that ends inside
+    a workgroup, and a head count that four do not divide."""
+    r = _case(num_tokens, num_heads, n_groups, tma, seed=3, dtype=dtype)
+    _check_bits(r, f"T={num_tokens} H={num_heads} tma={tma} {dtype}")
