@@ -838,8 +838,8 @@ int launch_gemm(const GemmArgs& a, void* workspace, size_t workspace_bytes, hipS
   const bool direct = (a.K > 0) && (a.K % 128 == 0) && (a.ldx % 16 == 0) && (a.ldw % 16 == 0) &&
                       (a.ldx < (1 << 23)) && (a.ldw < (1 << 23)) &&
                       ((uintptr_t)a.X % 16 == 0) && ((uintptr_t)a.W % 16 == 0);
-  // up to 128 rows: both operands through LDS, the weights read once (where that is the faster one: plan_skinny); the kernels below take
-  // the rest, and calls without the workspace that a split K needs
+  // up to 128 rows, and more where one round of blocks does them: deep stages of both operands through LDS (where that is the faster one:
+  // plan_skinny); the kernels below take the rest, and calls without the workspace that a split K needs
   if (direct && a.batch <= 1) {
     const SkinnyPlan sk = plan_skinny(a.M, a.N, a.K, MODE == kModeBlock);
     if (sk.use && (MODE != kModeBlock || skinny_takes_scales(a, sk)) &&

@@ -255,11 +255,11 @@ MidMPlan plan_mid_m(int64_t M, int64_t N, int64_t K, int64_t entries = 1);
 int launch_mid_m(const GemmArgs& a, int mode, const MidMPlan& plan, void* workspace, size_t workspace_bytes,
                  hipStream_t stream);
 
-// Up to 128 rows, fp8_gemm_skinny.hip: both operands through LDS in deep stages, the weights read once.
+// Up to 128 rows, or tiles for one round of blocks, fp8_gemm_skinny.hip: both operands through LDS in deep stages.
 struct SkinnyPlan {
   bool use;
   int cfg;                       // tile and ring (kShapes)
-  int tiles_n;                   // tiles along N
+  int tiles_n, tiles_m;          // tiles along N, rows of tiles
   int splits, stages_per_split;  // blocks along K, and the 256-byte stages of each
   size_t workspace_bytes;
 };

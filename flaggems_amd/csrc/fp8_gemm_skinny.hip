@@ -1,5 +1,5 @@
-// FP8 GEMM for up to 128 activation rows on gfx950: one row of tiles, 16 ... 128 rows x 32, 64 or 128 weight rows, both operands
-// through LDS in a ring of deep stages.
+// FP8 GEMM for few activation rows, or few tiles, on gfx950: tiles of 16 ... 128 rows x 32, 64 or 128 weight rows, both operands
+// through LDS in a ring of deep stages; up to 128 rows one row of tiles, beyond that as many tiles as fill the chip once.
 //
 // What bounds it: the weight stream out of HBM.  A compute unit gets about 85 GB/s out of its L2 and 49 GB/s when the lines
 // come from HBM, whatever is in flight beyond 40 KB, so the weights have to be spread over all units and the activations
@@ -31,7 +31,7 @@ namespace {
 
 struct SkinnyArgs {
   GemmArgs g;
-  int tiles_n, splits;
+  int tiles_n, tiles_m, splits;
   int stages_per_split;  // stages of 256 bytes of K per block
   int table_row;         // block mode: floats of a row of the scale table in LDS (odd), or 0: the table is [K-block][row]
   uint32_t table_row_magic;  // ceil(2^32 / table_row): quotients of entry numbers below 2^16 by multiplication
@@ -93,8 +93,20 @@ __global__ __launch_bounds__(2 * WM* WN * 64) void fp8_gemm_skinny_kernel(Skinny
   const int wm0 = (gw % WM) * (BM / WM), wn0 = (gw / WM) * (BN / WN);
   const int l16 = lane & 15, lg = lane >> 4;
 
-  const int tile = (int)blockIdx.x / a.splits, split = (int)blockIdx.x - tile * a.splits;
-  const int n0 = tile * BN;
+  // blocks of a split tile next to each other; with several rows of tiles, those against the same weights on one XCD (ids congruent
+  // mod 8), whose L2 then has the weights after the first of them
+  int tile, split, tile_m = 0;
+  if (a.tiles_m == 1) {
+    tile = (int)blockIdx.x / a.splits;
+    split = (int)blockIdx.x - tile * a.splits;
+  } else {
+    const int share = (int)gridDim.x >> 3, rem = (int)gridDim.x & 7, xcd = (int)blockIdx.x & 7;
+    const int at = xcd * share + (xcd < rem ? xcd : rem) + ((int)blockIdx.x >> 3), column = at / a.tiles_m;
+    tile_m = at - column * a.tiles_m;
+    split = column / a.tiles_n;
+    tile = column - split * a.tiles_n;
+  }
+  const int n0 = tile * BN, m0 = tile_m * BM, rows = g.M - m0 < BM ? g.M - m0 : BM;
   const int stages_all = (g.KB + 1) >> 1;
   const int s_begin = split * a.stages_per_split;
   const int stages = (stages_all - s_begin < a.stages_per_split) ? stages_all - s_begin : a.stages_per_split;  // >= 1
@@ -116,16 +128,16 @@ __global__ __launch_bounds__(2 * WM* WN * 64) void fp8_gemm_skinny_kernel(Skinny
   }
 #pragma unroll
   for (int j = 0; j < Cfg::kLoadsX; ++j) {
-    const int r = (wave + j * kWaves) * 4 + (lane >> 4), rc = r < g.M ? r : g.M - 1;
+    const int r = (wave + j * kWaves) * 4 + (lane >> 4), rc = r < rows ? r : rows - 1;
     x_off[j] = (uint32_t)rc * (uint32_t)g.ldx + (uint32_t)(chunk * 16);
   }
   // slabs of activations this wavefront copies: those past the last row stay as they are (a result depends on its own row)
-  const int slabs_x = (g.M + 3) / 4 < Cfg::kSlabsX ? (g.M + 3) / 4 : Cfg::kSlabsX;
+  const int slabs_x = (rows + 3) / 4;
   const int loads_x = slabs_x > wave ? (slabs_x - wave + kWaves - 1) / kWaves : 0;
   // a stage that ends after its first K-block re-reads that instead of the bytes past K
   const uint32_t back = (chunk & 8) ? 128u : 0u;
   const uint8_t* const w_base = uniform_ptr(g.W + (int64_t)n0 * g.ldw + (int64_t)kb0 * 128);
-  const uint8_t* const x_base = uniform_ptr(g.X + (int64_t)kb0 * 128);
+  const uint8_t* const x_base = uniform_ptr(g.X + (int64_t)m0 * g.ldx + (int64_t)kb0 * 128);
   auto issue_stage = [&](int s, int slot) __attribute__((always_inline)) {
     const uint32_t sub = s == half_stage ? back : 0u;
     const uint32_t dst = lds_base + (uint32_t)(slot * Cfg::kStageBytes);
@@ -148,14 +160,13 @@ __global__ __launch_bounds__(2 * WM* WN * 64) void fp8_gemm_skinny_kernel(Skinny
   // (rows an odd number of floats apart: 16 rows of a K-block lie in 16 banks), else with the rows next to each other
   const int t_row = a.table_row ? a.table_row : 1, t_kb = a.table_row ? 1 : BM;
   if (MODE == kModeBlock) {
-    const float* const xs_base = uniform_ptr(g.xs + (int64_t)kb0 * g.xs_cs);
+    const float* const xs_base = uniform_ptr(g.xs + (int64_t)m0 * g.xs_rs + (int64_t)kb0 * g.xs_cs);
     const int entries = a.table_row ? a.table_row * BM : kbs * BM;
     for (int i0 = wave * 64; i0 < entries; i0 += NT) {
       const uint32_t i = (uint32_t)(i0 + lane);
       int row = a.table_row ? (int)__umulhi(i, a.table_row_magic) : (int)(i % BM);
       int kb = a.table_row ? (int)i - row * a.table_row : (int)(i / BM);
-      row = row < BM ? row : BM - 1;
-      row = row < g.M ? row : g.M - 1;
+      row = row < rows ? row : rows - 1;
       kb = kb < kbs ? kb : kbs - 1;
       const uint32_t off = (uint32_t)(row * (int)g.xs_rs + kb * (int)g.xs_cs) * 4u;  // the host checks that this fits
       skinny_copy_4(off, xs_base, lds_base + (uint32_t)(Cfg::kRingBytes + i0 * 4));
@@ -280,16 +291,17 @@ __global__ __launch_bounds__(2 * WM* WN * 64) void fp8_gemm_skinny_kernel(Skinny
 
   // ---- K split over blocks: publish, count in, and let the wavefront that arrives last add the splits in order
   if (a.splits > 1) {
+    const int id = tile * a.tiles_m + tile_m;
     const uint32_t t_off = (uint32_t)tid * 16u;
     constexpr int kSlotFloats = kOwn * NT * 4;
-    float* const slots = uniform_ptr(a.partials + (size_t)tile * a.splits * kSlotFloats);
+    float* const slots = uniform_ptr(a.partials + (size_t)id * a.splits * kSlotFloats);
     {
       float* const mine = uniform_ptr(slots + (size_t)split * kSlotFloats);
 #pragma unroll
       for (int q = 0; q < kOwn; ++q) store_x4_agent(mine + q * NT * 4, t_off, own[q]);
     }
     wait_vmem_all();
-    unsigned int* const cnt = a.counters + tile * kWaves + wave;
+    unsigned int* const cnt = a.counters + id * kWaves + wave;
     unsigned int prev = 0;
     if (lane == 0) prev = __hip_atomic_fetch_add(cnt, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     prev = (unsigned int)__builtin_amdgcn_readfirstlane((int)prev);
@@ -320,12 +332,12 @@ __global__ __launch_bounds__(2 * WM* WN * 64) void fp8_gemm_skinny_kernel(Skinny
     if (lane == 0) __hip_atomic_store(cnt, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);  // ready for the next launch
   }
 
-  // ---- results: the lane holds m = wm0 + j * 16 + l16, n = n0 + wn0 + i * 16 + 4 * lg + [0, 4)
+  // ---- results: the lane holds m = m0 + wm0 + j * 16 + l16, n = n0 + wn0 + i * 16 + 4 * lg + [0, 4)
 #pragma unroll
   for (int q = 0; q < kOwn; ++q) {
     const int t = kItems > 1 && group ? q + kOwn : q;
     const int i = t / TM, j = t % TM;
-    const int m = wm0 + j * 16 + l16;
+    const int m = m0 + wm0 + j * 16 + l16;
     if (m < g.M) store_output4<MODE>(g, m, n0 + wn0 + i * 16 + lg * 4, own[q]);
   }
 }
@@ -342,7 +354,7 @@ int launch_skinny_cfg(SkinnyArgs sa, const SkinnyPlan& plan, int mode, hipStream
                                                   reinterpret_cast<const void*>(kr), reinterpret_cast<const void*>(ki));
     if (e != hipSuccess) FG_FAIL(FG_ERR_LAUNCH, "hipFuncSetAttribute(%d bytes LDS): %s", Cfg::kLdsBytes, hipGetErrorString(e));
   }
-  const dim3 grid((uint32_t)(plan.tiles_n * plan.splits)), block(Cfg::kThreads);
+  const dim3 grid((uint32_t)(sa.tiles_n * sa.tiles_m * sa.splits)), block(Cfg::kThreads);
   if (mode == kModeBlock) FG_LAUNCH(kb, grid, block, Cfg::kLdsBytes, stream, sa);
   else if (mode == kModeRowColI8) FG_LAUNCH(ki, grid, block, Cfg::kLdsBytes, stream, sa);
   else FG_LAUNCH(kr, grid, block, Cfg::kLdsBytes, stream, sa);
@@ -369,6 +381,15 @@ constexpr SkinnyShape kShapes[] = {
     {64, 64, 4, 8, 3.85f, 0.215f, 0.205f, 11.3f, 2.73f, 1.52f, 0.94f},
     {64, 128, 3, 8, 4.96f, 0.276f, 0.216f, 8.9f, 4.52f, 2.29f, 1.22f},
     {128, 64, 3, 8, 4.88f, 0.139f, 0.434f, 8.0f, 3.59f, 2.22f, 1.55f},
+};
+// The same for several rows of tiles (7100 problems of 129 to 1000 rows): the weights come out of HBM once for all rows of tiles, so
+// less of the time is the stream and more of it the stages.
+constexpr int kFirstOfRows = 6;
+constexpr SkinnyShape kShapesOfRows[] = {
+    {64, 32, 3, 4, 4.07f, 0.18f, 0.06f, 7.92f, 1.84f, 1.82f, 0.08f},
+    {64, 64, 4, 8, 4.01f, 0.32f, 0.17f, 17.1f, 2.51f, 1.30f, 1.03f},
+    {64, 128, 3, 8, 4.89f, 0.41f, 0.29f, 16.0f, 3.65f, 2.76f, 1.21f},
+    {128, 64, 3, 8, 5.23f, 0.39f, 0.28f, 23.3f, 3.66f, 2.10f, 1.66f},
 };
 
 float skinny_cost(const SkinnyShape& sh, int64_t M, int64_t N, int64_t K, int64_t tiles, int64_t per, int64_t splits, int cus) {
@@ -404,9 +425,18 @@ bool skinny_table_fits(const SkinnyShape& sh, int64_t stages) {
 //    8192 rows with K past 6144 do better on 128 x 128 tiles (128, 28672 x 4096: 34.8 -> 34.9; 104, 9664 x 13440 +23 %), and so do weights that one
 //    block's scales do not cover in the split that suits them (96, 7168 x 16384: 39 -> 46 in five parts); short K against 3072 to 4096
 //    weight rows does better in two parts (104, 3072 x 2048: 9.0 -> 10.0).
+//  * 129 to 1000 rows, in one round of blocks: 17.4 -> 13.8 (256, 4096 x 4096), 15.8 -> 12.3 (200, 7168 x 2304), 36.6 -> 31.4 (256, 8192 x 8192,
+//    row and column scales), 10.3 -> 5.7 (600, 896 x 896); geometric mean of 3090 problems 0.70.  Two rounds lose (333, 8192 x 8192 +25 %), and so
+//    does a longer K against the persistent kernel's tiles shared along K: more than 80 tiles of 128 x 64 (597, 1664 x 5632: 18.3 -> 20.8; 256,
+//    5120 x 7552: 24.8 -> 31.2), more than 40 (701, 704 x 14976: 24.4 -> 35.7), more than 160 past 8192 or past 512 rows (512, 4096 x 14336: 46.5 ->
+//    73.7; 628, 2112 x 7168: 24.0 -> 28.1; block scales from 7424: 252, 5376 x 7424: 25.6 -> 29.9).  Against few weight rows the parts of up to 16 rows are ahead (192, 512 x 2816: 5.1 -> 7.3; 200, 768 x
+//    3840: 7.3 -> 8.9; 200, 832 x 1792: 5.8 -> 6.4; 426, 512 x 1152: 4.5 -> 5.1).
+//  * past 1000 rows: up to 2048 with K to 3072 (1280, 1600 x 1024: 14.4 -> 10.1), or to 4608 against 768 weight rows and fewer (geometric mean
+//    0.75; 1942, 384 x 5120: 17.9 -> 21.3; wider ones 0.95 with +15 to +27 % in every tenth); past 2048 K to 2560 (0.65 to 0.73; to 5632 0.93,
+//    every tenth +15 %).
 SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales) {
   SkinnyPlan p = {};
-  if (M < 1 || M > 128 || N < 512 || K < 512 || K % 128 != 0) return p;
+  if (M < 1 || M > 4096 || N < (M > 1000 ? 128 : 512) || K < 512 || K % 128 != 0) return p;
   const int cus = cu_count();
   const int64_t stages = (K / 128 + 1) / 2, bytes = N * K, mb = 1000000;
   int best = -1;
@@ -424,16 +454,20 @@ SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales) {
     best_per = stages;
   } else {
     bool use = M <= 64 && K < 1024;
+    const int64_t units = ceil_div(M * N, (int64_t)8192);  // tiles of 128 x 64
     if (M <= 32) use = use || N > 6144 || (N > 4096 && (bytes <= 16 * mb || bytes >= 48 * mb)) || (N > 3072 && bytes >= 40 * mb) || (N >= 1024 && K >= 11008 && M * K >= 240000);
     else if (M <= 64) use = use || N >= 4096 || (N > 3072 && bytes >= 8 * mb) || (N >= 2048 && bytes >= 20 * mb) || (N >= 1536 && K >= 11008);
-    else use = N <= 16384 && (N >= 8192 ? K <= 6144 : N > 4096 ? K >= 1024 : N >= 3072 ? K >= 3072 : (N >= 2048 && K >= 6144));
+    else if (M <= 128) use = N <= 16384 && (N >= 8192 ? K <= 6144 : N > 4096 ? K >= 1024 : N >= 3072 ? K >= 3072 : (N >= 2048 && K >= 6144));
+    else if (M <= 1000) use = units <= cus && (K <= 5120 || units <= 40 || (units <= 80 && K <= 8192) || (M <= 512 && K <= (block_scales ? 7168 : 8192) && units > 160)) &&
+                              !(M <= 256 && N <= 1024 && bytes <= (N <= 768 ? 6 : 2) * mb) && !(M <= 512 && N <= 512 && bytes <= 2 * mb);
+    else use = units <= cus && (M <= 2048 ? K <= 3072 || (K <= 4608 && N <= 768) : K <= 2560);
     if (!use) return p;
-    const int first = M <= 16 ? 0 : M <= 32 ? 3 : M <= 64 ? 6 : 9, last = M <= 64 ? first + 3 : 10;
+    const int first = M <= 16 ? 0 : M <= 32 ? 3 : M <= 64 ? 6 : M <= 128 ? 9 : kFirstOfRows, last = M <= 64 ? first + 3 : 10;
     float best_cost = 0.f, any_cost = 0.f;
-    bool any_fits = true;
+    bool any_fits = true, one_round = true;
     for (int c = first; c < last; ++c) {
-      const SkinnyShape& sh = kShapes[c];
-      const int64_t tiles = ceil_div(N, (int64_t)sh.bn);
+      const SkinnyShape& sh = M > 128 ? kShapesOfRows[c - kFirstOfRows] : kShapes[c];
+      const int64_t tiles = ceil_div(N, (int64_t)sh.bn) * ceil_div(M, (int64_t)sh.bm);
       int64_t seen = 0;
       for (int64_t s = 1; s <= 12 && (s == 1 || tiles * s * 2 <= (int64_t)cus * 9); ++s) {
         const int64_t per = ceil_div(stages, s), splits = ceil_div(stages, per);
@@ -443,18 +477,22 @@ SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales) {
         const float cost = skinny_cost(sh, M, N, K, tiles, per, splits, cus);
         const bool fits = !block_scales || skinny_table_fits(sh, per);
         if (any_cost == 0.f || cost < any_cost) { any_cost = cost; any_fits = fits; }
-        if (fits && (best < 0 || cost < best_cost)) { best = c; best_per = per; best_cost = cost; }
+        if (fits && (best < 0 || cost < best_cost)) {
+          best = c; best_per = per; best_cost = cost;
+          one_round = tiles * splits <= (sh.waves == 4 ? 2 : 1) * (int64_t)cus;
+        }
       }
     }
-    if (best < 0 || (M > 64 && !any_fits)) return p;
+    if (best < 0 || (M > 64 && M <= 128 && !any_fits) || (M > 128 && !one_round)) return p;
   }
   const SkinnyShape& sh = kShapes[best];
   p.cfg = best;
   p.tiles_n = (int)ceil_div(N, (int64_t)sh.bn);
+  p.tiles_m = (int)ceil_div(M, (int64_t)sh.bm);
   p.stages_per_split = (int)best_per;
   p.splits = (int)ceil_div(stages, best_per);
   const int64_t items = (int64_t)sh.bm * sh.bn / 256 / (sh.waves / 2), own = items > 1 ? items / 2 : 1;
-  p.workspace_bytes = p.splits > 1 ? FG_WORKSPACE_COUNTER_BYTES + (size_t)p.tiles_n * p.splits * own * sh.waves * 64 * 16 : 0;
+  p.workspace_bytes = p.splits > 1 ? FG_WORKSPACE_COUNTER_BYTES + (size_t)p.tiles_n * p.tiles_m * p.splits * own * sh.waves * 64 * 16 : 0;
   p.use = true;
   return p;
 }
@@ -471,6 +509,7 @@ int launch_skinny(const GemmArgs& g, int mode, const SkinnyPlan& plan, void* wor
   SkinnyArgs sa = {};
   sa.g = g;
   sa.tiles_n = plan.tiles_n;
+  sa.tiles_m = plan.tiles_m;
   sa.splits = plan.splits;
   sa.stages_per_split = plan.stages_per_split;
   if (mode == kModeBlock) {

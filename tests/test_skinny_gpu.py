@@ -1,4 +1,4 @@
-"""The kernel for up to 128 rows (csrc/fp8_gemm_skinny.hip): every tile shape at the fewest and most rows it takes, weights that
+"""The kernel for few rows or few tiles (csrc/fp8_gemm_skinny.hip): every tile shape at the fewest and most rows it takes, weights that
 end inside a tile, odd and even numbers of K-blocks (the last stage holds one), K in one range and split, both layouts of the
 activation scales, every result and operand type."""
 import pytest
@@ -20,6 +20,14 @@ _SHAPES = [
     (33, 7105, 1152), (64, 4097, 8064), (63, 28609, 1152), (64, 7168, 16384), (33, 2100, 9856), (48, 1600, 11008), (61, 640, 512),
     # 128 rows a tile
     (65, 3073, 1152), (128, 14337, 1152), (127, 4100, 7552), (97, 2112, 7168),
+    # several rows of tiles, the last of one row, of a part and full: 64 x 32
+    (1001, 128, 512), (4096, 129, 896), (321, 577, 5248), (449, 512, 8064), (1001, 128, 2688),
+    # 64 x 64
+    (193, 2049, 512), (130, 3073, 2560), (129, 2100, 5248), (257, 1537, 5120), (191, 1537, 12288),
+    # 64 x 128
+    (193, 4100, 512), (257, 6209, 7168), (321, 3073, 896), (129, 2049, 7168), (257, 2049, 8192),
+    # 128 x 64
+    (193, 4100, 2688), (513, 3073, 2560), (1000, 577, 8192), (385, 1537, 8064),
 ]
 
 
@@ -67,9 +75,9 @@ def test_rows_past_the_last_do_not_reach_the_result():
     N, K = 8192, 4096
     w = torch.randn(N, K, device=DEV).to(torch.float8_e4m3fn)
     ws = torch.ones(N // 128, K // 128, device=DEV)
-    nan = torch.full((128, K), float("nan"), device=DEV).to(torch.float8_e4m3fn)
-    for rows in (1, 17, 33, 65):
+    nan = torch.full((256, K), float("nan"), device=DEV).to(torch.float8_e4m3fn)
+    for rows in (1, 17, 33, 65, 193):
         x = torch.randn(rows, K, device=DEV).to(torch.float8_e4m3fn)
-        flag_gems.w8a8_block_fp8_matmul(nan, w, torch.ones(128, K // 128, device=DEV), ws, [128, 128])
+        flag_gems.w8a8_block_fp8_matmul(nan, w, torch.ones(256, K // 128, device=DEV), ws, [128, 128])
         got = flag_gems.w8a8_block_fp8_matmul(x, w, torch.ones(rows, K // 128, device=DEV), ws, [128, 128])
         assert not got.isnan().any()
