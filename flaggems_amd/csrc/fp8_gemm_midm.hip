@@ -1,5 +1,5 @@
-// FP8 GEMM for 33 <= M <= 64 activation rows on gfx950 (and more rows against small weights, in parts of up to 64): the weight is
-// read once, straight from global memory into MFMA operand registers, and the activations come out of LDS.
+// FP8 GEMM for 33 <= M <= 64 activation rows on gfx950 (and more rows against small weights, in parts of up to 64), where the
+// kernel of fp8_gemm_skinny.hip is not the faster one or cannot take the call: the weight is read once, straight from global memory into MFMA operand registers, and the activations come out of LDS.
 //
 // With up to 64 rows the activation slice of a K-block (64 x 128 bytes) is as large as the 64 weight rows a
 // wavefront multiplies it with, so a wavefront that fetches both from global memory moves two bytes for every
