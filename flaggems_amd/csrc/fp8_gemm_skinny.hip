@@ -416,6 +416,10 @@ bool skinny_table_fits(const SkinnyShape& sh, int64_t stages) {
 //    means of 60 to 160 problems a cell allow: 32-row tiles, block scales, K to 6144 0.92-0.98 (row and column scales 0.97-1.02); 64-row tiles,
 //    block scales 0.87-0.96, row and column scales to 6144 0.93-0.99, past it 1.00-1.04; 128-row tiles, block scales 4096 to 8192 0.85-0.91 (2048
 //    to 4096 1.02-1.04), row and column scales 0.89-1.01 (2048 to 4096 and past 8192 1.00-1.06).
+//  * 9 to 16 rows, block scales, K split: long K against up to 1536 weight rows 0.92 (9, 1536 x 14080: 14.7 -> 8.4; 768 and fewer 0.98), past 16384
+//    up to 2560 0.85 (13, 1920 x 17664: 13.9 -> 10.1; up to 12 rows only to 1344: 11, 1472 x 19584 10.2 -> 12.2), and 3585 to 4096 0.93 (16, 4096 x 14336: 15.2 -> 13.8; up to 12 rows with a shorter K 0.97,
+//    a quarter of them 3-12 % slower).  In between the activations of the decode kernels fit LDS in ranges that fill the units (10, 2112 x 10240: 7.9 -> 9.4;
+//    9, 3072 x 9216: +20 %); row and column scales 1.02.
 //  * 17 to 32 rows: 36.6 -> 26.3 (32, 7168 x 16384), 32.4 -> 23.4 (32, 28672 x 4096), 23.2 -> 14.5 (32, 8192 x 8192); up to 6144 weight
 //    rows the parts of up to 16 rows are ahead in between (20, 3968 x 6272: 8.4 -> 11.1; 17, 4608 x 7168: 12.2 -> 13.4) and where their activations
 //    still fit LDS (18, 1344 x 11264: 7.9 -> 8.8).
@@ -441,7 +445,9 @@ SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales) {
   const int64_t stages = (K / 128 + 1) / 2, bytes = N * K, mb = 1000000;
   int best = -1;
   int64_t best_per = 0;
-  if (M <= 16 && K >= 1024) {
+  const bool narrow_long = block_scales && M > 8 && M <= 16 && ((N <= (M > 12 ? 2560 : 1344) && K > 16384) || (N > 768 && N <= 1536 && K > 9216 && K <= 16384) ||
+                                                                (N > 3584 && N <= 4096 && (K >= 14336 || (M > 12 && K > 10240))));
+  if (M <= 16 && K >= 1024 && !narrow_long) {
     for (int c = 0; c < 3; ++c) {
       const int64_t tiles = ceil_div(N, (int64_t)kShapes[c].bn);
       if (tiles <= cus && tiles * 4 > (int64_t)cus * 3) best = c;
@@ -453,7 +459,7 @@ SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales) {
     if (!far_rows && !(use && M > 8)) return p;
     best_per = stages;
   } else {
-    bool use = M <= 64 && K < 1024;
+    bool use = (M <= 64 && K < 1024) || narrow_long;
     const int64_t units = ceil_div(M * N, (int64_t)8192);  // tiles of 128 x 64
     if (M <= 32) use = use || N > 6144 || (N > 4096 && (bytes <= 16 * mb || bytes >= 48 * mb)) || (N > 3072 && bytes >= 40 * mb) || (N >= 1024 && K >= 11008 && M * K >= 240000);
     else if (M <= 64) use = use || N >= 4096 || (N > 3072 && bytes >= 8 * mb) || (N >= 2048 && bytes >= 20 * mb) || (N >= 1536 && K >= 11008);
@@ -483,7 +489,7 @@ SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales) {
         }
       }
     }
-    if (best < 0 || (M > 64 && M <= 128 && !any_fits) || (M > 128 && !one_round)) return p;
+    if (best < 0 || ((M > 64 || (M <= 16 && K >= 1024)) && M <= 128 && !any_fits) || (M > 128 && !one_round)) return p;
   }
   const SkinnyShape& sh = kShapes[best];
   p.cfg = best;

@@ -14,6 +14,8 @@ _STEP = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.
 _SHAPES = [
     # 16 rows a tile: 32, 64 and 128 weight rows; short K, one round that fills the units
     (1, 512, 512), (16, 4097, 640), (5, 577, 896), (9, 6209, 1152), (16, 12353, 1152), (16, 24641, 1152), (3, 28672, 4096), (1, 8192, 4096),
+    # K split
+    (9, 833, 9344), (16, 1536, 14080), (13, 2500, 16512), (16, 4096, 14336), (13, 3585, 10368), (9, 513, 16512),
     # 32 rows a tile
     (17, 8129, 1152), (32, 12290, 1280), (31, 28609, 1152), (17, 1030, 14336), (32, 4100, 14464), (20, 3000, 768),
     # 64 rows a tile
