@@ -34,6 +34,23 @@ def test_host_tensors_are_left_to_the_general_path():
         h.connect(1, 2)
 
 
+def test_the_modules_bring_no_thread_local_storage():
+    """A module with a thread-local segment that nothing touches makes every access to the thread-local storage of the libraries
+    loaded before it slow (glibc before 2.39): all other host work of the process, by a sixth."""
+    import struct
+
+    from flaggems_amd.build import fastcall_path, hostcalls_path
+
+    for path in (fastcall_path(), hostcalls_path()):
+        with open(path, "rb") as f:
+            data = f.read()
+        assert data[:6] == b"\x7fELF\x02\x01"
+        offset, = struct.unpack_from("<Q", data, 32)
+        size, count = struct.unpack_from("<HH", data, 54)
+        kinds = [struct.unpack_from("<I", data, offset + i * size)[0] for i in range(count)]
+        assert 1 in kinds and 7 not in kinds, path  # PT_LOAD, PT_TLS
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("rows,cols,pad", [(1, 128, 0), (5, 384, 0), (7, 1024, 64), (1, 256, 32), (300, 7168, 0)])
