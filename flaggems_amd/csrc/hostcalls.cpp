@@ -56,7 +56,10 @@ int type_code(ScalarType t) {  // FG_BF16, FG_F16, FG_F32
   return t == ScalarType::BFloat16 ? 0 : t == ScalarType::Half ? 1 : t == ScalarType::Float ? 2 : -1;
 }
 
-bool is_128(PyObject* o) { return PyLong_CheckExact(o) && PyLong_AsLong(o) == 128; }
+bool is_128(PyObject* o) {
+  int beyond = 0;  // (a number that fits no long is no error here: the Python code refuses it)
+  return PyLong_CheckExact(o) && PyLong_AsLongAndOverflow(o, &beyond) == 128;
+}
 
 // The workspace a problem asks for depends on its sizes alone; the last sizes asked are remembered (under the GIL).
 size_t workspace_bytes(int64_t m, int64_t n, int64_t k) {

@@ -30,6 +30,10 @@ def test_host_tensors_are_left_to_the_general_path():
     assert h.block_matmul(a, a, a, a, 128, 128, torch.bfloat16, False) is None
     assert h.group_quant(a, 128, False, 1e-10, 0, 1, 0) is None
     assert h.block_matmul(None, 1, "x", a, 128, 128, torch.bfloat16, False) is None
+    for beyond in (2 ** 70, -(2 ** 70)):  # fits no long: no error left behind
+        assert h.block_matmul(a, a, a, a, beyond, 128, torch.bfloat16, False) is None
+        assert h.block_matmul(a, a, a, a, 128, beyond, torch.bfloat16, False) is None
+        assert h.group_quant(a, beyond, False, 1e-10, 0, 1, 0) is None
     with pytest.raises(TypeError):
         h.connect(1, 2)
 
