@@ -268,9 +268,9 @@ _ws_bytes_cache = {}
 
 
 def cached_workspace_bytes(fn_name: str, *shape) -> int:
-    """``lib.<fn_name>(*shape)``, remembered per shape (the answer depends on the shape and the device's compute unit
-    count only; processes that mix GPU models would have to clear the table)."""
-    key = (fn_name, shape)
+    """``lib.<fn_name>(*shape)``, remembered per shape and current device (the answer depends on the shape and the device's
+    compute unit count only)."""
+    key = (fn_name, shape) if _single_gpu is not False else (fn_name, shape, torch.cuda.current_device())
     n = _ws_bytes_cache.get(key)
     if n is None:
         n = int(getattr(load(), fn_name)(*shape))

@@ -61,13 +61,15 @@ bool is_128(PyObject* o) {
   return PyLong_CheckExact(o) && PyLong_AsLongAndOverflow(o, &beyond) == 128;
 }
 
-// The workspace a problem asks for depends on its sizes alone; the last sizes asked are remembered (under the GIL).
-size_t workspace_bytes(int64_t m, int64_t n, int64_t k) {
-  static struct { int64_t m, n, k; size_t bytes; } seen[64] = {};
+// The workspace a problem asks for depends on its sizes and on the current device's compute units alone; the last ones asked are
+// remembered (under the GIL).
+size_t workspace_bytes(int64_t m, int64_t n, int64_t k, int device) {
+  static struct { int64_t m, n, k; int device; size_t bytes; } seen[64] = {};
   auto& e = seen[(uint64_t)(m * 31 + n * 7 + (k >> 7)) % 64];
-  if (e.m != m || e.n != n || e.k != k) {
+  if (e.m != m || e.n != n || e.k != k || e.device != device) {
     e.bytes = gemm_workspace(m, n, k);
     e.m = m; e.n = n; e.k = k;
+    e.device = device;
   }
   return e.bytes;
 }
@@ -103,7 +105,7 @@ PyObject* block_matmul(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (pow2 < 0) return nullptr;
   Tensor c = at::empty({m, n}, a->options().dtype(out));
   if (!plain(c)) Py_RETURN_NONE;  // (a mode that makes other tensors)
-  const size_t bytes = workspace_bytes(m, n, k);
+  const size_t bytes = workspace_bytes(m, n, k, device.index());
   void* ws = nullptr;
   size_t ws_len = 0;
   THPObjectPtr ws_tensor;

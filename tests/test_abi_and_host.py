@@ -192,6 +192,26 @@ def test_batched_workspace_query_is_host_only_and_never_below_the_single_problem
     assert lib.fg_batched_block_fp8_gemm_workspace_bytes(16, 64, 1024, 7168) > lib.fg_block_fp8_gemm_workspace_bytes(64, 1024, 7168)
 
 
+def test_workspace_sizes_are_remembered_per_device(monkeypatch):
+    """The planners ask the current device for its compute units: what one device needs is no answer for another."""
+    class Library:
+        asked = 0
+
+        def sizes(self, m, n):
+            self.asked += 1
+            return 1000 * torch.cuda.current_device() + m + n
+
+    library, device = Library(), [0]
+    monkeypatch.setattr(_lib, "load", lambda: library)
+    monkeypatch.setattr(_lib, "_ws_bytes_cache", {})
+    monkeypatch.setattr(_lib, "_single_gpu", False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: device[0])
+    for _ in range(2):
+        for device[0] in (0, 1, 2):
+            assert _lib.cached_workspace_bytes("sizes", 3, 4) == 1000 * device[0] + 7
+    assert library.asked == 3
+
+
 def test_group_ends_from_the_per_block_expert_table():
     """expert_ids as the reference's moe_align_block_size lays it out (one entry per block of sorted rows, experts
     ascending, -1 past the padded end) -> cumulative row ends per expert."""
