@@ -255,15 +255,8 @@ MidMPlan plan_mid_m(int64_t M, int64_t N, int64_t K, int64_t entries = 1);
 int launch_mid_m(const GemmArgs& a, int mode, const MidMPlan& plan, void* workspace, size_t workspace_bytes,
                  hipStream_t stream);
 
-// Up to 128 rows, or tiles for one round of blocks, fp8_gemm_skinny.hip: both operands through LDS in deep stages.
-struct SkinnyPlan {
-  bool use;
-  int cfg;                       // tile and ring (kShapes)
-  int tiles_n, tiles_m;          // tiles along N, rows of tiles
-  int splits, stages_per_split;  // blocks along K, and the 256-byte stages of each
-  size_t workspace_bytes;
-};
-SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales);
+// Up to 128 rows, or tiles for one round of blocks, fp8_gemm_skinny.hip (fp8_gemm_skinny_plan.h says which).
+struct SkinnyPlan;
 bool skinny_takes_scales(const GemmArgs& a, const SkinnyPlan& plan);
 int launch_skinny(const GemmArgs& a, int mode, const SkinnyPlan& plan, void* workspace, hipStream_t stream);
 

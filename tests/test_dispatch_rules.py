@@ -1,4 +1,4 @@
-"""The hand-over rules of csrc/fp8_gemm_rules.h against measurements on an MI355X (256 compute units): shapes on both sides of every
+"""The hand-over rules of csrc/fp8_gemm_rules.h and csrc/fp8_gemm_skinny_plan.h against measurements on an MI355X (256 compute units): shapes on both sides of every
 line, with the time of either kernel, so that a rule that moves a line has to answer for them.  Host code only."""
 import ctypes
 import os
@@ -7,9 +7,10 @@ import subprocess
 
 import pytest
 
-HEADER = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flaggems_amd", "csrc", "fp8_gemm_rules.h")
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "flaggems_amd", "csrc")
 SHIM = """
-#include "%s"
+#include "%s/fp8_gemm_rules.h"
+#include "%s/fp8_gemm_skinny_plan.h"
 extern "C" int tall(int block, long long M, long long N, long long kb, long long cus) { return fg::tall_tiles_pay(block != 0, M, N, kb, cus); }
 extern "C" int stream_rows(long long M, long long N, long long kb, long long groups, long long cus) {
   return fg::grouped_stream_pass_rows(M, N, kb, groups, cus);
@@ -20,7 +21,13 @@ extern "C" int parts(long long M, long long N, long long K, long long* rows, lon
   return (int)d.parts;
 }
 extern "C" int copy_rows(long long M, long long N, long long K, long long groups, long long cus) { return fg::gather_copy_pays(M, N, K, groups, cus); }
-""" % HEADER
+extern "C" int skinny(int block, long long M, long long N, long long K, int cus, int* plan) {
+  const fg::SkinnyPlan p = fg::plan_skinny(M, N, K, block != 0, cus);
+  if (!p.use) return 0;
+  plan[0] = fg::kSkinnyShapes[p.cfg].bm, plan[1] = fg::kSkinnyShapes[p.cfg].bn, plan[2] = p.tiles_m, plan[3] = p.splits;
+  return 1;
+}
+""" % (CSRC, CSRC)
 
 
 @pytest.fixture(scope="module")
@@ -36,8 +43,38 @@ def rules(tmp_path_factory):
     so = ctypes.CDLL(lib)
     so.tall.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
     so.stream_rows.argtypes = so.copy_rows.argtypes = [ctypes.c_longlong] * 5
+    so.skinny.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 3 + [ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     so.parts.argtypes = [ctypes.c_longlong] * 3 + [ctypes.POINTER(ctypes.c_longlong)] * 2
     return so
+
+
+def _skinny(rules, block, M, N, K):
+    """(rows a tile, weight rows a tile, rows of tiles, parts of K), or None where another kernel takes the problem."""
+    plan = (ctypes.c_int * 4)()
+    return tuple(plan) if rules.skinny(block, M, N, K, 256, plan) else None
+
+
+@pytest.mark.parametrize("block", [True, False])
+def test_the_shapes_of_the_deep_stage_kernels_tests_reach_every_form_of_it(rules, block):
+    import test_skinny_gpu as T
+
+    forms, rows = set(), {}
+    for M, N, K in T.BLOCK_SCALES if block else T.ROW_AND_COLUMN_SCALES:
+        plan = _skinny(rules, block, M, N, K)
+        assert plan is not None, (M, N, K)
+        bm, bn, tiles_m, splits = plan
+        forms.add((bm, bn, tiles_m > 1, splits > 1, K // 128 % 2))
+        if tiles_m == 1:
+            rows.setdefault((bm, bn), []).append(M)
+    tiles = [(bm, bn) for bm in (16, 32, 64) for bn in (32, 64, 128)] + [(128, 64)]
+    for bm, bn in tiles:
+        for several in (False, True) if bm >= 64 else (False,):
+            for split in (False, True) if block or bm > 16 else (False,):
+                for odd in (0, 1):
+                    assert (bm, bn, several, split, odd) in forms
+        assert min(rows[bm, bn]) == (1 if bm == 16 else bm // 2 + 1) and max(rows[bm, bn]) >= bm - 1
+    if block:
+        assert {_skinny(rules, True, *shape)[:2] for shape in T._EVERY_TILE} == set(tiles)
 
 
 def test_parts_of_the_rows_stay_inside_the_matrix(rules):
