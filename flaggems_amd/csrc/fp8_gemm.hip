@@ -842,7 +842,7 @@ int launch_gemm(const GemmArgs& a, void* workspace, size_t workspace_bytes, hipS
   // up to 128 rows, and more where one round of blocks does them: deep stages of both operands through LDS (where that is the faster one:
   // plan_skinny); the kernels below take the rest, and calls without the workspace that a split K needs
   if (direct && a.batch <= 1) {
-    const SkinnyPlan sk = plan_skinny(a.M, a.N, a.K, MODE == kModeBlock, cu_count());
+    const SkinnyPlan sk = plan_skinny(a.M, a.N, a.K, a.ldw, MODE == kModeBlock, cu_count());
     if (sk.use && (MODE != kModeBlock || skinny_takes_scales(a, sk)) &&
         (sk.splits == 1 || (workspace != nullptr && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= sk.workspace_bytes)))
       return launch_skinny(a, MODE, sk, workspace, stream);
@@ -1020,7 +1020,7 @@ extern "C" size_t fg_block_fp8_gemm_workspace_bytes(int64_t M, int64_t N, int64_
     }
   }
   for (const bool block_scales : {false, true}) {
-    const fg::SkinnyPlan sk = fg::plan_skinny(M, N, K, block_scales, fg::cu_count());
+    const fg::SkinnyPlan sk = fg::plan_skinny(M, N, K, K, block_scales, fg::cu_count());
     if (sk.use && sk.workspace_bytes > need) need = sk.workspace_bytes;
   }
   const size_t pp = fg::pingpong_workspace_bytes(M, N, K);

@@ -70,14 +70,21 @@ inline bool skinny_table_fits(const SkinnyShape& sh, int64_t stages) {
   return (skinny_div((kbs | 1) * sh.bm, 64) * 64 + skinny_div(kbs, 64) * 64) * 4 <= room;
 }
 
-// Where this kernel is the faster one (us, the kernels of the other files -> this one, both with their best split; M rows, N x K):
+// Where this kernel is the faster one (us, the kernels of the other files -> this one, both with their best split; M rows, N x K; `ldw`: bytes
+// from one weight row to the next, which decides only where K is not split, so that no workspace depends on it):
 //  * up to 64 rows, K of 512 to 896: always (28, 4096 x 896: 5.6 -> 4.2; 16, 11584 x 896: 6.0 -> 4.5).
 //  * up to 16 rows, K from 1024: unsplit in one round that fills over three quarters of the units; emptier rounds lose (12, 9216 x 5120:
-//    12.0 -> 13.2).  Where the weight's rows lie 4 or 8 KB apart the other kernels' blocks meet on few memory channels: 24.9 -> 22.3 (1,
-//    28672 x 4096), 27.8 -> 22.8 (16), 16.2 -> 13.6 (1, 8192 x 8192), 15.5 -> 12.7 (16, 14336 x 4096).  Otherwise from 9 rows, with the K that geometric
-//    means of 60 to 160 problems a cell allow: 32-row tiles, block scales, K to 6144 0.92-0.98 (row and column scales 0.97-1.02); 64-row tiles,
-//    block scales 0.87-0.96, row and column scales to 6144 0.93-0.99, past it 1.00-1.04; 128-row tiles, block scales 4096 to 8192 0.85-0.91 (2048
-//    to 4096 1.02-1.04), row and column scales 0.89-1.01 (2048 to 4096 and past 8192 1.00-1.06).
+//    12.0 -> 13.2).  What pays depends on the tile, on K and on how far apart the weight's rows lie (`ldw`): 4 or 8 KB apart, the other kernels'
+//    blocks meet on few memory channels.  Geometric means over 25600 problems of 1 to 16 rows, by the tile's weight rows:
+//     - 128: K = 4096 0.85-0.90 (16, 28672 x 4096: 27.8 -> 22.8; with rows 4224 bytes apart 1.04-1.11: 3, 30656: 21.3 -> 23.8), 8192 from 9
+//       rows 0.86-0.98 (1, 30272: 41.0 -> 44.6, row and column scales); from 9 rows, K in between 0.87-0.97 and, row and column scales, below 1920 0.95
+//       (2048 to 4095 1.01-1.05).
+//     - 64: K = 4096 0.81-0.95 (4, 14848: 14.8 -> 12.6), 8192 0.82-0.96 (row and column scales up to 8 rows 1.00); from 9 rows, block scales to 10240
+//       0.76-0.96 (13, 15872 x 2048: 9.1 -> 8.3), past it 0.97 (up to 12 rows 10241 to 10752 and from 12416 on 0.98-1.06: 9, 16128 x 14336: 38.9 ->
+//       41.4); row and column scales to 1280 0.87-0.93, to 4096 from 13 rows 0.98 (up to 12 rows 1.00: 10, 15936 x 3584: 12.0 -> 12.7; past it 1.01-1.10).
+//     - 32: block scales from 9 rows, to 4096 0.95, to 6144 from 13 rows 0.98 (up to 12 rows 1.00: 9, 6400 x 4480: 8.0 -> 8.3; rows 8 KB apart: 15,
+//       6272 x 4096: 8.4 -> 8.9); 8192, and 4096 with block scales, from 13 rows (14, 6976 x 8192: 13.7 -> 13.3) or in a round over 15/16 full (12,
+//       8192 x 8192: 16.6 -> 13.5); otherwise 1.00-1.15 (10, 6464 x 8192: 11.7 -> 12.6).
 //  * 9 to 16 rows, block scales, K split: long K against up to 1536 weight rows 0.92 (9, 1536 x 14080: 14.7 -> 8.4; 768 and fewer 0.98), past 16384
 //    up to 2560 0.85 (13, 1920 x 17664: 13.9 -> 10.1; up to 12 rows only to 1344: 11, 1472 x 19584 10.2 -> 12.2), and 3585 to 4096 0.93 (16, 4096 x 14336: 15.2 -> 13.8; up to 12 rows with a shorter K 0.97,
 //    a quarter of them 3-12 % slower).  In between the activations of the decode kernels fit LDS in ranges that fill the units (10, 2112 x 10240: 7.9 -> 9.4;
@@ -88,7 +95,8 @@ inline bool skinny_table_fits(const SkinnyShape& sh, int64_t stages) {
 //  * 33 to 64 rows: 40.7 -> 28.5 (61, 7168 x 16384), 22.8 -> 16.3 (61, 4096 x 14336), 16.8 -> 12.8 (61, 4608 x 7168), 32.9 -> 25.0 (61,
 //    28672 x 4096); narrow weights only if they are long or large (64, 1280 x 5120: 4.8 -> 7.7 against sixteen-row parts).
 //  * 65 to 128 rows: 20.5 -> 16.5 (96, 4608 x 7168), 28 -> 20.8 (80, 4096 x 14336), 33 -> 23 (80, 14336 x 4096); weights of more than
-//    8192 rows with K past 6144 do better on 128 x 128 tiles (128, 28672 x 4096: 34.8 -> 34.9; 104, 9664 x 13440 +23 %), and so do weights that one
+//    8192 rows with K past 6144 do better on 128 x 128 tiles, as do, with row and column scales, 5121 to 6656 with long K and many rows (117, 5504 x
+//    16128: 32.6 -> 35.9; 103, 5824 x 16000: 31.5 -> 33.9) (128, 28672 x 4096: 34.8 -> 34.9; 104, 9664 x 13440 +23 %), and so do weights that one
 //    block's scales do not cover in the split that suits them (96, 7168 x 16384: 39 -> 46 in five parts); short K against 3072 to 4096
 //    weight rows does better in two parts (104, 3072 x 2048: 9.0 -> 10.0).
 //  * 129 to 1000 rows, in one round of blocks: 17.4 -> 13.8 (256, 4096 x 4096), 15.8 -> 12.3 (200, 7168 x 2304), 36.6 -> 31.4 (256, 8192 x 8192,
@@ -100,7 +108,7 @@ inline bool skinny_table_fits(const SkinnyShape& sh, int64_t stages) {
 //  * past 1000 rows: up to 2048 with K to 3072 (1280, 1600 x 1024: 14.4 -> 10.1), or to 4608 against 768 weight rows and fewer (geometric mean
 //    0.75; 1942, 384 x 5120: 17.9 -> 21.3; wider ones 0.95 with +15 to +27 % in every tenth); past 2048 K to 2560 (0.65 to 0.73; to 5632 0.93,
 //    every tenth +15 %).
-inline SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales, int cus) {
+inline SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, int64_t ldw, bool block_scales, int cus) {
   SkinnyPlan p = {};
   if (M < 1 || M > 4096 || N < (M > 1000 ? 128 : 512) || K < 512 || K % 128 != 0) return p;
   const int64_t stages = (K / 128 + 1) / 2, bytes = N * K, mb = 1000000;
@@ -114,16 +122,27 @@ inline SkinnyPlan plan_skinny(int64_t M, int64_t N, int64_t K, bool block_scales
       if (tiles <= cus && tiles * 4 > (int64_t)cus * 3) best = c;
     }
     if (best < 0 || (block_scales && !skinny_table_fits(kSkinnyShapes[best], stages))) return p;
-    // (up to 8 rows with the shortest tiles only in a full round: 3, 6208 x 8192: 10.9 -> 12.1)
-    const bool far_rows = K % 4096 == 0 && K <= 8192 && (best > 0 || M > 8 || skinny_div(N, (int64_t)kSkinnyShapes[0].bn) * 16 > (int64_t)cus * 15);
-    const bool use = best == 0 ? block_scales && K <= 6144 : best == 1 ? block_scales || K <= 6144 : K <= 8192 && (block_scales ? K >= 4096 : K < 2048 || K >= 4096);
-    if (!far_rows && !(use && M > 8)) return p;
+    // the weight's rows lie next to each other; 4 KB apart or a multiple; begin inside a cache line
+    const bool own = ldw == K, apart = ldw % 4096 == 0, torn = ldw % 128 != 0;
+    const bool full = skinny_div(N, (int64_t)kSkinnyShapes[0].bn) * 16 > (int64_t)cus * 15;
+    bool use;
+    if (best == 0) {
+      use = (own && K % 4096 == 0 && K <= 8192 && (block_scales || K == 8192) && (M > 12 || full)) ||
+            (block_scales && M > 8 && K <= (M > 12 ? 6144 : 4096) && (own || ldw % 8192 != 0));
+    } else if (best == 1) {
+      use = ((apart || torn) && (K == 4096 || (K == 8192 && (block_scales || M > 8)))) ||
+            (M > 8 && (block_scales ? M > 12 || K <= 10240 || (K > 10752 && K <= 12288) || K % 4096 == 0 : K <= 1280 || (M > 12 && K <= 4096 && (own || !apart))));
+    } else {
+      use = ((apart || torn) && (K == 4096 || (K == 8192 && M > 8))) || (M > 8 && ((K > 4096 && K <= 8192) || (!block_scales && K < 1920)));
+    }
+    if (!use) return p;
     best_per = stages;
   } else {
     bool use = (M <= 64 && K < 1024) || narrow_long;
     const int64_t units = skinny_div(M * N, (int64_t)8192);  // tiles of 128 x 64
     if (M <= 32) use = use || N > 6144 || (N > 4096 && (bytes <= 16 * mb || bytes >= 48 * mb)) || (N > 3072 && bytes >= 40 * mb) || (N >= 1024 && K >= 11008 && M * K >= 240000);
     else if (M <= 64) use = use || N >= 4096 || (N > 3072 && bytes >= 8 * mb) || (N >= 2048 && bytes >= 20 * mb) || (N >= 1536 && K >= 11008);
+    else if (M <= 128 && !block_scales && N > 5120 && N <= 6656 && M * K > 1180000) use = false;
     else if (M <= 128) use = N <= 16384 && (N >= 8192 ? K <= 6144 : N > 4096 ? K >= 1024 : N >= 3072 ? K >= 3072 : (N >= 2048 && K >= 6144));
     else if (M <= 1000) use = units <= cus && (K <= 5120 || units <= 40 || (units <= 80 && K <= 8192) || (M <= 512 && K <= (block_scales ? 7168 : 8192) && units > 160)) &&
                               !(M <= 256 && N <= 1024 && bytes <= (N <= 768 ? 6 : 2) * mb) && !(M <= 512 && N <= 512 && bytes <= 2 * mb);

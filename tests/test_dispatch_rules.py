@@ -21,8 +21,8 @@ extern "C" int parts(long long M, long long N, long long K, long long* rows, lon
   return (int)d.parts;
 }
 extern "C" int copy_rows(long long M, long long N, long long K, long long groups, long long cus) { return fg::gather_copy_pays(M, N, K, groups, cus); }
-extern "C" int skinny(int block, long long M, long long N, long long K, int cus, int* plan) {
-  const fg::SkinnyPlan p = fg::plan_skinny(M, N, K, block != 0, cus);
+extern "C" int skinny(int block, long long M, long long N, long long K, long long ldw, int cus, int* plan) {
+  const fg::SkinnyPlan p = fg::plan_skinny(M, N, K, ldw, block != 0, cus);
   if (!p.use) return 0;
   plan[0] = fg::kSkinnyShapes[p.cfg].bm, plan[1] = fg::kSkinnyShapes[p.cfg].bn, plan[2] = p.tiles_m, plan[3] = p.splits;
   return 1;
@@ -43,15 +43,15 @@ def rules(tmp_path_factory):
     so = ctypes.CDLL(lib)
     so.tall.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4
     so.stream_rows.argtypes = so.copy_rows.argtypes = [ctypes.c_longlong] * 5
-    so.skinny.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 3 + [ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
+    so.skinny.argtypes = [ctypes.c_int] + [ctypes.c_longlong] * 4 + [ctypes.c_int, ctypes.POINTER(ctypes.c_int)]
     so.parts.argtypes = [ctypes.c_longlong] * 3 + [ctypes.POINTER(ctypes.c_longlong)] * 2
     return so
 
 
-def _skinny(rules, block, M, N, K):
+def _skinny(rules, block, M, N, K, ldw=None):
     """(rows a tile, weight rows a tile, rows of tiles, parts of K), or None where another kernel takes the problem."""
     plan = (ctypes.c_int * 4)()
-    return tuple(plan) if rules.skinny(block, M, N, K, 256, plan) else None
+    return tuple(plan) if rules.skinny(block, M, N, K, ldw or K, 256, plan) else None
 
 
 @pytest.mark.parametrize("block", [True, False])
@@ -75,6 +75,34 @@ def test_the_shapes_of_the_deep_stage_kernels_tests_reach_every_form_of_it(rules
         assert min(rows[bm, bn]) == (1 if bm == 16 else bm // 2 + 1) and max(rows[bm, bn]) >= bm - 1
     if block:
         assert {_skinny(rules, True, *shape)[:2] for shape in T._EVERY_TILE} == set(tiles)
+
+
+# block scales?, M, N, K, bytes from one weight row to the next, us on the deep-stage kernel, us on the kernel that serves the shape otherwise
+DEEP = [
+    # 32 weight rows a tile: K = 8192 from 13 rows or in a nearly full round; block scales from 9 rows with short K
+    (False, 9, 6592, 8192, 8192, 12.9, 11.8), (False, 10, 6464, 8192, 8192, 12.6, 11.7), (False, 11, 6656, 8192, 8192, 12.7, 12.0),
+    (False, 10, 7488, 8192, 8192, 13.7, 13.1), (False, 16, 7232, 8192, 8192, 13.6, 14.0), (False, 14, 6976, 8192, 8192, 13.3, 13.7),
+    (False, 12, 8192, 8192, 8192, 13.5, 16.6), (False, 7, 6720, 4096, 4096, 7.9, 7.4), (False, 5, 8000, 4096, 4096, 8.8, 8.1),
+    (True, 9, 6400, 4480, 4480, 8.3, 8.0),
+    # 64: K = 4096, 8192; longer K with block scales from 13 rows
+    (False, 7, 15680, 4096, 4096, 13.4, 14.4), (True, 8, 15552, 4096, 4096, 13.0, 15.4), (True, 15, 12352, 2048, 2048, 7.3, 8.3),
+    (True, 9, 16128, 14336, 14336, 41.4, 38.9), (True, 11, 12352, 14336, 14336, 34.2, 33.4), (False, 10, 15936, 3584, 3584, 12.7, 12.0),
+    (False, 10, 15552, 5120, 5120, 17.0, 16.0), (False, 14, 14464, 1024, 1024, 5.3, 6.1),
+    # 128
+    (False, 1, 30272, 8192, 8192, 44.6, 41.0), (True, 13, 32128, 4096, 4096, 24.4, 28.8),
+    # rows that lie as far apart as another K's, or K's rows further apart
+    (False, 3, 16128, 4096, 4224, 13.8, 13.2), (False, 3, 29056, 4096, 4224, 22.8, 20.4), (False, 8, 25472, 4096, 4224, 20.6, 19.2),
+    (True, 14, 30976, 4096, 5120, 24.0, 22.8), (True, 12, 30080, 4096, 4224, 23.0, 21.7), (True, 9, 27648, 4096, 4128, 22.4, 33.8),
+    (False, 11, 6720, 4096, 8192, 9.2, 8.0), (True, 15, 6272, 4096, 8192, 8.9, 8.4), (True, 14, 13888, 2048, 2176, 7.7, 8.8),
+    # many rows, long K, row and column scales
+    (False, 117, 5504, 16128, 16128, 35.9, 32.6), (False, 114, 5632, 16384, 16384, 35.5, 32.1), (False, 103, 5824, 16000, 16000, 33.9, 31.5),
+    (False, 71, 5504, 14592, 14592, 27.7, 28.6),
+]
+
+
+@pytest.mark.parametrize("block,M,N,K,ldw,deep,other", DEEP)
+def test_deep_stage_kernel_where_it_is_the_faster_one(rules, block, M, N, K, ldw, deep, other):
+    assert (_skinny(rules, block, M, N, K, ldw) is not None) == (deep < other)
 
 
 def test_parts_of_the_rows_stay_inside_the_matrix(rules):

@@ -43,7 +43,7 @@ BLOCK_SCALES = [
 ]
 # (rows of the result are multiples of 16 bytes here; 16 rows a tile are not split along K)
 ROW_AND_COLUMN_SCALES = [
-    (1, 512, 512), (16, 4112, 640), (5, 592, 896), (1, 8192, 4096), (16, 8176, 8192),
+    (1, 512, 512), (16, 4112, 640), (5, 592, 896), (9, 8192, 8192), (16, 8176, 8192),
     (16, 12368, 1152), (1, 8208, 512),
     (16, 24656, 1152), (3, 28672, 4096), (1, 24672, 4096),
     (17, 8144, 1152), (32, 7120, 768), (20, 3008, 768), (17, 1040, 14336), (22, 1040, 11392),
