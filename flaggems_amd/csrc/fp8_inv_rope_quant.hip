@@ -185,7 +185,6 @@ int launch_inv_rope(const InvRopeArgs& a, int64_t padded_tokens, hipStream_t str
   const int64_t pieces = ceil_div(padded_tokens, (int64_t)kRopeTokens) * a.heads;
   const int hpw = XDT != FG_F32 && pieces >= 4864 && a.heads % 4 == 0 ? 4 : pieces >= (XDT == FG_F32 ? 2400 : 2048) && a.heads % 2 == 0 ? 2 : 1;
   const int64_t head_blocks = a.heads / hpw, blocks = pieces / hpw;
-  if (blocks > 0x7FFFFFFF) FG_FAIL(FG_ERR_UNSUPPORTED, "fg_inv_rope_group_quant_fp8: too many workgroups");
   const dim3 grid((uint32_t)blocks), block(kRopeThreads);
   auto go = [&](auto plain, auto packed) { FG_LAUNCH(a.packed ? packed : plain, grid, block, 0, stream, a, (int)padded_tokens, (int)head_blocks); };
   if (hpw == 4) go(inv_rope_quant_kernel<XDT, LPG, XDT == FG_F32 ? 2 : 4, false>, inv_rope_quant_kernel<XDT, LPG, XDT == FG_F32 ? 2 : 4, true>);
@@ -253,7 +252,22 @@ extern "C" int fg_inv_rope_group_quant_fp8(const void* o, int o_dtype, int64_t t
   a.qa.floor = eps; a.qa.lo = -448.0f; a.qa.hi = 448.0f; a.qa.inv_max = 1.0f / 448.0f;
   a.qa.scale_rule = FG_SCALE_MUL_INV; a.qa.quotient_rule = FG_QUOT_DIV;
   a.qa.pow2_rule = pack_ue8m0 ? FG_POW2_LOG2 : FG_POW2_NONE; a.qa.e5m2 = 0;
-  if (o_dtype == FG_BF16) return launch_inv_rope_group<FG_BF16>(a, padded_tokens, (hipStream_t)stream);
-  if (o_dtype == FG_F16) return launch_inv_rope_group<FG_F16>(a, padded_tokens, (hipStream_t)stream);
-  return launch_inv_rope_group<FG_F32>(a, padded_tokens, (hipStream_t)stream);
+  // A launch counts its threads in 32 bits, 2^24 workgroups of 256: 2^26 heads, 8 GB of them at 64 values each.  Longer calls go out in runs of
+  // tokens (a whole number of workgroups each).
+  const int64_t run = ((int64_t)1 << 23) / heads * kRopeTokens;
+  for (int64_t t = 0; t < padded_tokens; t += run) {
+    InvRopeArgs r = a;
+    r.o = reinterpret_cast<const char*>(o) + t * o_stride_token * esz;
+    r.positions = reinterpret_cast<const char*>(positions) + t * position_bytes;
+    r.q = a.q + t * q_stride_token;
+    r.s = reinterpret_cast<uint32_t*>(scales) + t;
+    const int64_t left = padded_tokens - t, padded = left < run ? left : run;
+    r.tokens = (int)(tokens - t < padded ? (tokens > t ? tokens - t : 0) : padded);
+    int rc;
+    if (o_dtype == FG_BF16) rc = launch_inv_rope_group<FG_BF16>(r, padded, (hipStream_t)stream);
+    else if (o_dtype == FG_F16) rc = launch_inv_rope_group<FG_F16>(r, padded, (hipStream_t)stream);
+    else rc = launch_inv_rope_group<FG_F32>(r, padded, (hipStream_t)stream);
+    if (rc != FG_OK) return rc;
+  }
+  return FG_OK;
 }

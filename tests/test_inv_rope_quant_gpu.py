@@ -278,3 +278,18 @@ def test_heads_a_wavefront_takes(num_tokens, num_heads, n_groups, tma, dtype):
     a workgroup, and a head count that four do not divide."""
     r = _case(num_tokens, num_heads, n_groups, tma, seed=3, dtype=dtype)
     _check_bits(r, f"T={num_tokens} H={num_heads} tma={tma} {dtype}")
+
+
+def test_more_workgroups_than_a_launch_takes_along_one_dimension():
+    """2^28 heads and more, one of each token repeated: the first and the last tokens are those of small calls."""
+    tokens, heads = (1 << 22) + 6, 64
+    base = torch.randn(tokens, 1, 64, device=DEV, dtype=torch.bfloat16)
+    positions = torch.arange(tokens, device=DEV, dtype=torch.int32) % 512
+    cache = torch.randn(512, 64, device=DEV)
+    take = lambda part: flag_gems.fused_inv_rope_fp8_quant(  # noqa: E731
+        base[part].expand(-1, heads, -1), positions[part], cache, 1, heads, nope_dim=0, rope_dim=64, quant_group_size=64)
+    codes, scales = take(slice(None))
+    for first in (0, (1 << 20) - 3, tokens - 5):
+        part = slice(first, first + 5)
+        few, few_scales = take(part)
+        assert torch.equal(codes[part].view(torch.uint8), few.view(torch.uint8)) and torch.equal(scales[part], few_scales)
