@@ -743,6 +743,8 @@ PipePlan plan_pipe(bool block_scales, int64_t M, int64_t N, int64_t K, int64_t x
   // with up to 128 K-blocks per block allowed here: M = 1024, N = 4096, K = 14336: 74 -> 82 us; with up to 64: M = 512,
   // same weights: 53 -> 45 us; N = 7168, K = 16384 at M = 256: 59 -> 50 us).
   if (p.kb_per_split > 64) return p;
+  // (Up to 64 rows of a lone problem come here only where the deep-stage kernel cannot take the call: a split K without its workspace,
+  // or scales too far apart for 32-bit offsets.  The figures below compare the kernels that are left then.)
   // 33..64 rows: half of every tile is padding, and so is half of every partial tile a split writes; the
   // staged-activation kernel is the alternative.  This kernel wins while K is split in two at most over ranges of
   // eight K-blocks or more (measured at M = 64: N = 28672, K = 4096, 224 tiles unsplit: 46 -> 32 us; N = 24576, K = 1536:
@@ -922,12 +924,15 @@ int launch_gemm(const GemmArgs& a, void* workspace, size_t workspace_bytes, hipS
     // against 16.8 -- and only serves batches now)
     const bool mid_takes = mid.use && mid.tmx <= 4;
     if (a.M > 16 && a.M <= 48) {
-      // very wide weights against short K: a wavefront per 16 weight rows with the block's activations in LDS
+      // very wide weights against a K of 128 to 384 (longer ones: plan_skinny): a wavefront per 16 weight rows with the block's activations
+      // in LDS
       // (N = 24576, K = 1536, M = 17 / 24 / 32 / 40: 15.1 / 13.8 / 13.7 / 14.2 us on the kernels below)
       const SmallMPlan sp = plan_small_m(a.M, a.N, a.K);
       if (sp.use && sp.own) return launch_small_m(a, MODE, sp, workspace, workspace_bytes, stream);
     }
-    if (a.M <= 64) {  // the four-stage tile kernel where its planner prefers it to the staged-activation and decode kernels
+    // calls that the deep-stage kernel could not take: the four-stage tile kernel where its planner prefers it to the staged-activation and
+    // decode kernels
+    if (a.M <= 64) {
       const PipePlan pp = plan_pipe(MODE == kModeBlock, a.M, a.N, a.K, MODE == kModeBlock ? a.xs_rs : 0);
       const bool ws_ok = pp.splits == 1 || (workspace != nullptr && workspace_bytes >= pp.workspace_bytes && (uintptr_t)workspace % 16 == 0);
       if (pp.use && ws_ok) return launch_pipe<MODE>(a, pp, workspace, stream);

@@ -71,9 +71,8 @@ def test_quantized_linear_shapes_bf16(M, N, K):
 @pytest.mark.parametrize("M", [17, 24, 25, 32, 40, 64])
 @pytest.mark.parametrize("N,K", [(24576, 1536), (28672, 4096), (14336, 4096)])
 def test_few_rows_against_wide_weights(M, N, K):
-    """17 ... 64 rows against weights wide enough to give every compute unit a 128 x 128 tile (or half the units one, with
-    K in two ranges) leave the decode and staged-activation kernels for the four-stage tile kernel: all of them against
-    the oracle, whichever kernel the planner picks for the row count."""
+    """17 ... 64 rows against weights wide enough to give every compute unit a tile of the deep-stage kernel, which takes all
+    of these: against the oracle."""
     xq, wq, xs, ws = _quantized_inputs(M, N, K, seed=M)
     want = O.block_fp8_matmul_dequant_ref(xq, wq, xs, ws, [128, 128], torch.float32, torch.float64)
     got = flag_gems.w8a8_block_fp8_matmul(xq.to(DEV), wq.to(DEV), xs.to(DEV), ws.to(DEV), [128, 128])
@@ -107,9 +106,8 @@ def test_persistent_kernel_several_rounds_ragged_edges_and_strides():
 @pytest.mark.parametrize("M,N,K", [(100, 520, 2048), (128, 1300, 4096), (48, 384, 8192)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_few_tiles_split_along_k(M, N, K, dtype):
-    """32 < M <= 128 with a handful of 128 x 128 tiles: the tile kernel splits K over blocks and the last
-    wavefront of a tile adds the partial sums in split order.  Against the oracle in every output type, and
-    bit-identical on reruns."""
+    """32 < M <= 128 against weights of few rows: the decode kernels in parts of up to 16 rows, K split over blocks and the
+    partial sums added in split order.  Against the oracle in every output type, and bit-identical on reruns."""
     xq, wq, xs, ws = _quantized_inputs(M, N, K, seed=9)
     want = O.block_fp8_matmul_dequant_ref(xq, wq, xs, ws, [128, 128], torch.float32, torch.float64)
     args = (xq.to(DEV), wq.to(DEV), xs.to(DEV), ws.to(DEV), [128, 128])
@@ -125,8 +123,8 @@ def test_few_tiles_split_along_k(M, N, K, dtype):
 @pytest.mark.parametrize("M,N,K", [(2048, 512, 2048), (1300, 1000, 2304), (4096, 384, 1024), (3000, 1100, 896)])
 def test_tall_problems_against_narrow_weights(M, N, K):
     """More than 1024 rows but at most one 128 x 128 tile per compute unit: the four-stage tile kernel with K split
-    over blocks, not the persistent kernel.  Ragged M and N, 7 and 18 K-blocks; against the oracle and bit-identical
-    on reruns."""
+    over blocks ((3000, 1100, 896)) or, with K of up to 2560 in one round of its tiles, the deep-stage kernel (the others), not the
+    persistent kernel.  Ragged M and N, 7 and 18 K-blocks; against the oracle and bit-identical on reruns."""
     xq, wq, xs, ws = _quantized_inputs(M, N, K, seed=23)
     want = O.block_fp8_matmul_dequant_ref(xq, wq, xs, ws, [128, 128], torch.float32, torch.float64)
     args = (xq.to(DEV), wq.to(DEV), xs.to(DEV), ws.to(DEV), [128, 128])
@@ -141,10 +139,9 @@ def test_tall_problems_against_narrow_weights(M, N, K):
                                    (500, 260, 8192), (512, 1000, 1152), (256, 1100, 4096), (300, 4100, 512)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_129_to_512_rows_against_tiny_weights(M, N, K, dtype):
-    """Weights of a few MB: the kernel of 33 to 64 rows takes the rows in three to eight equal parts in one launch (the
-    last part with fewer rows), each part reading the weights again ((200, 1030, 4096), (256, 2048, 2048), (190, 1280, 8192),
-    (256, 1100, 4096), (300, 4100, 512)); against the very smallest the decode kernels take sixteen or thirty-two parts
-    of up to 16 rows (the others).  Ragged M and N, column-major activation scales; against the oracle and bit-identical
+    """Weights of a few MB: the decode kernels take fifteen to thirty-two parts of up to 16 rows against the very smallest
+    ((129, 576, 7168) and (500, 260, 8192)), each part reading the weights again; the others are one round of the deep-stage
+    kernel's tiles, K in one range or split.  Ragged M and N, column-major activation scales; against the oracle and bit-identical
     on reruns."""
     xq, wq, xs, ws = _quantized_inputs(M, N, K, seed=29)
     want = O.block_fp8_matmul_dequant_ref(xq, wq, xs, ws, [128, 128], torch.float32, torch.float64)
@@ -187,18 +184,13 @@ def test_129_to_512_tiles_of_128_rows(M, N, K, dtype):
                                    (40, 2112, 7168), (64, 1536, 12288), (35, 8192, 1536), (100, 1000, 8192), (128, 2048, 2048), (77, 1536, 7168)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 def test_33_to_128_rows(M, N, K, dtype):
-    """33 <= M <= 64 (and 65 <= M <= 128 with small weights) takes the kernel that keeps the activations in LDS and
-    streams the weights (wide weights with up to 48 rows: a wavefront per 16 weight rows, the second line of shapes): one K range or several (partial sums added in split order), N that ends inside a 16-row
-    group, fewer rows than are staged, every output type, column-major scales; against the oracle and bit-identical
-    on reruns.  The last line of shapes: that kernel's blocks would leave a second round of compute units mostly idle,
-    so the four-stage tile kernel takes them with K in three and four ranges; the last shape has 131 tiles, which that kernel
-    splits in three ranges rather than leave half of the compute units idle; the two after it are too wide for one round of tiles
-    and run in rounds of blocks whose K split is chosen by how full the rounds are; the last five (and (65, 520, 1024),
-    (100, 2112, 4096), (128, 4096, 4096) above) have 65 to 128 rows against small weights, which the same kernel takes as two
-    halves of the rows in one launch (48 or 64 rows staged, a second half with fewer rows than the first); the last two lines are
-    33 to 64 rows against weights of up to 13 MB (26 MB when narrow), which the decode kernels take in four parts of up to 16
-    rows that share rows where the count does not divide, and 65 to 128 rows against weights of up to 11.5 MB in eight parts
-    ((50, 8200, 1024) is just too wide for that and stays on the staged-activation kernel)."""
+    """33 to 128 rows: the deep-stage kernel where the weights have some width and K some length, else the decode kernels in
+    four or eight parts of up to 16 rows that share rows where the count does not divide (33 to 64 rows against weights of up to
+    13 MB, 26 MB when narrow; 65 to 128 against up to 11.5 MB), the kernel that keeps the activations in LDS and streams the
+    weights, in two halves of the rows ((81, 3000, 4224)), or the four-stage tile kernel, 131 tiles in three ranges of K
+    ((70, 16650, 8192)).  K in one range and split, N that ends inside a tile, fewer rows than a tile has, every output type,
+    column-major scales; against the oracle and bit-identical on reruns.  (tests/test_skinny_gpu.py sends calls of these sizes past the
+    deep-stage kernel to the others.)"""
     xq, wq, xs, ws = _quantized_inputs(M, N, K, seed=13)
     want = O.block_fp8_matmul_dequant_ref(xq, wq, xs, ws, [128, 128], torch.float32, torch.float64)
     args = (xq.to(DEV), wq.to(DEV), xs.to(DEV), ws.to(DEV), [128, 128])
@@ -241,9 +233,11 @@ def test_up_to_32_rows_uneven_chunks(M, N, K, dtype):
     with 128 KB of activations or more (half the blocks on half of K each, the half ranges in LDS or in the two slots;
     the six shapes from (16, 2304, 16384) on and (9, 4096, 14336)), 17 to 32 rows against short K and few tiles
     ((24, 8192, 1024) and the next), 17 to 32 rows against weights of up to 6144 rows (two parts of up to 16 rows in one
-    launch, sharing the middle row when the count is odd: (20, 4608, 4096), (17, 2050, 1152), the three from
-    (17, 2304, 16384) on and the five from (21, 2112, 7168) on), column-major activation scales; against the oracle and
-    bit-identical on reruns."""
+    launch, sharing the middle row when the count is odd: (20, 4608, 4096), (17, 2050, 1152), and the five from
+    (21, 2112, 7168) on), column-major activation scales; against the oracle and bit-identical on reruns.  The deep-stage
+    kernel takes those of 17 rows and more against over 6144 weight rows or with K of 14336 and more, and (16, 32768, 512),
+    (16, 28672, 4096), (16, 8192, 8192), (9, 3590, 18944) and (9, 4096, 14336); tests/test_skinny_gpu.py sends such calls past it to the kernels
+    that the shapes were listed for."""
     xq, wq, xs, ws = _quantized_inputs(M, N, K, seed=17)
     want = O.block_fp8_matmul_dequant_ref(xq, wq, xs, ws, [128, 128], torch.float32, torch.float64)
     args = (xq.to(DEV), wq.to(DEV), xs.to(DEV), ws.to(DEV), [128, 128])

@@ -75,6 +75,9 @@ def test_the_shapes_of_the_deep_stage_kernels_tests_reach_every_form_of_it(rules
         assert min(rows[bm, bn]) == (1 if bm == 16 else bm // 2 + 1) and max(rows[bm, bn]) >= bm - 1
     if block:
         assert {_skinny(rules, True, *shape)[:2] for shape in T._EVERY_TILE} == set(tiles)
+        assert all(_skinny(rules, True, *shape)[3] > 1 for shape in T.WITHOUT_WORKSPACE)
+        assert sum(_skinny(rules, True, *shape) is not None for shape in T.SCALES_FAR_APART) >= 12
+        assert all(_skinny(rules, True, *shape) is None for shape in T.SHORT_K)
 
 
 # block scales?, M, N, K, bytes from one weight row to the next, us on the deep-stage kernel, us on the kernel that serves the shape otherwise

@@ -154,6 +154,46 @@ def test_rows_further_apart_than_they_are_long(M, N, K):
     assert (wide[:, :16] == 7.0).all() and (wide[:, 16 + N:] == 7.0).all()
 
 
+# what other kernels serve: calls without the workspace that a split K needs (up to 16 rows, and 33 to 64 against weights that those
+# kernels split too, such a call is refused), activation scales whose rows lie too far apart for
+# 32-bit offsets, and K below 512 against wide weights
+WITHOUT_WORKSPACE = [(17, 2304, 16384), (32, 3590, 18944), (24, 4096, 14336), (40, 19178, 8192), (65, 2112, 7168), (128, 4096, 4096), (128, 2048, 16384), (200, 1030, 4096), (190, 1280, 8192), (257, 1537, 5120)]
+SCALES_FAR_APART = [(9, 3590, 18944), (16, 28672, 4096), (16, 8192, 8192), (17, 24576, 1536), (32, 28672, 4096), (24, 16384, 1024), (20, 4608, 7168),
+                    (40, 24584, 1536), (33, 49152, 2048), (37, 16384, 1024), (48, 8330, 6144), (64, 6650, 8192), (50, 7168, 16384), (61, 4608, 7168)]
+SHORT_K = [(40, 16384, 384), (64, 20000, 256), (24, 24576, 384), (50, 10000, 128), (60, 12345, 384), (17, 30000, 256)]
+
+
+@pytest.mark.parametrize("M,N,K,how", [s + ("no workspace",) for s in WITHOUT_WORKSPACE] + [s + ("scales far apart",) for s in SCALES_FAR_APART] +
+                         [s + ("",) for s in SHORT_K])
+def test_calls_that_the_deep_stage_kernel_cannot_take(M, N, K, how):
+    from flaggems_amd import _lib
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.float8_e4m3fn)
+    w = (0.5 * torch.randn(N, K, generator=g, device=DEV)).to(torch.float8_e4m3fn)
+    xs = torch.rand(M, K // 128, generator=g, device=DEV) * 0.02 + 0.005
+    ws = torch.rand(-(-N // 128), K // 128, generator=g, device=DEV) * 0.02 + 0.005
+    a = x.float() * xs.repeat_interleave(128, 1)
+    b = w.float() * ws.repeat_interleave(128, 1).repeat_interleave(128, 0)[:N]
+    want, mag = a @ b.t(), a.abs() @ b.abs().t()
+    lib, dev = _lib.load(), torch.device(DEV)
+    if how == "scales far apart":
+        far = torch.zeros(M, 1 << 21, device=DEV)
+        far[:, :K // 128] = xs
+        xs = far[:, :K // 128]
+    for dtype in _STEP:
+        wsp = None if how == "no workspace" else _lib.workspace(dev, lib.fg_block_fp8_gemm_workspace_bytes(M, N, K))
+        got = []
+        for _ in range(2):
+            c = torch.full((M, N), 7.0, device=DEV, dtype=dtype)
+            rc = lib.fg_block_fp8_gemm(x.data_ptr(), K, w.data_ptr(), K, xs.data_ptr(), xs.stride(0), 1, ws.data_ptr(), ws.stride(0), 1, c.data_ptr(), N,
+                                       _lib.DTYPE_CODE[dtype], M, N, K, 128, 128, None if wsp is None else wsp.data_ptr(), 0 if wsp is None else wsp.numel(),
+                                       _lib.current_stream_ptr(dev))
+            _lib.check(rc, "fg_block_fp8_gemm")
+            got.append(c)
+        assert ((got[0].float() - want).abs() <= want.abs() * _STEP[dtype] + 4e-4 * mag).all()
+        assert torch.equal(*got)
+
+
 def test_rows_past_the_last_do_not_reach_the_result():
     # one row of a 16- and of a 64-row tile whose other rows are whatever the kernel before left in LDS: NaN codes
     N, K = 8192, 4096
