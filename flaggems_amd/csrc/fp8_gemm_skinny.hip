@@ -1,10 +1,15 @@
 // FP8 GEMM for few activation rows, or few tiles, on gfx950: tiles of 16 ... 128 rows x 32, 64 or 128 weight rows, both operands
 // through LDS in a ring of deep stages; up to 128 rows one row of tiles, beyond that as many tiles as fill the chip once.
 //
-// What bounds it: the weight stream out of HBM.  A compute unit gets about 85 GB/s out of its L2 and 49 GB/s when the lines
-// come from HBM, whatever is in flight beyond 40 KB, so the weights have to be spread over all units and the activations
-// that every unit fetches again have to stay few: with 64 x 128 tiles they are half as many bytes as the weights.  Copies to
-// LDS take whole lines (the fragment layout of the matrix instructions, 16 rows x 64 bytes a load, reaches a third of that).
+// What bounds it: the copies to LDS.  Alone, in this kernel's tiles, ring and order, a compute unit gets
+//    119 GB/s (50 B/clk)  all 256 units the same lines, which their L2s hold
+//     92                  216 tiles of 64 x 128 in six rows of tiles (333 rows, 4608 x 7168), weights left in the caches by the launch before
+//     58                  the same with the weights out of HBM, 1.4 TB/s of them (23.8 us of the product's 26); 61 for 128 x 64 in two rows
+//                         (256 rows, 8192 x 8192, 2.6 TB/s: 25.8 us)
+//     35                  no tile shares its weights: 256 units take 6 TB/s, which is HBM's rate
+// whatever is in flight beyond 40 KB.  So the weights have to be spread over all units, and the activations that every unit
+// fetches again have to stay few: with 64 x 128 tiles they are half as many bytes as the weights.  The copies take whole lines (the
+// fragment layout of the matrix instructions, 16 rows x 64 bytes a load, reaches a third of that).
 //
 //  * A stage is 256 bytes of K (two K-blocks) of every row: four rows an instruction, each 256 bytes in a run.  The
 //    wavefronts form two groups; group g multiplies K-block 2 s + g of stage s.  One barrier per stage, that is per two
