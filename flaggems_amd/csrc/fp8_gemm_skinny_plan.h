@@ -71,7 +71,8 @@ inline bool skinny_table_fits(const SkinnyShape& sh, int64_t stages) {
 }
 
 // Where this kernel is the faster one (us, the kernels of the other files -> this one, both with their best split; M rows, N x K; `ldw`: bytes
-// from one weight row to the next, which decides only where K is not split, so that no workspace depends on it):
+// from one weight row to the next, which decides only where K is not split, so that no workspace depends on it).  Measured on 256 compute
+// units, which the lines in M, N and K are for; rounds and splits follow the units that there are.
 //  * up to 64 rows, K of 512 to 896: always (28, 4096 x 896: 5.6 -> 4.2; 16, 11584 x 896: 6.0 -> 4.5).
 //  * up to 16 rows, K from 1024: unsplit in one round that fills over three quarters of the units; emptier rounds lose (12, 9216 x 5120:
 //    12.0 -> 13.2).  What pays depends on the tile, on K and on how far apart the weight's rows lie (`ldw`): 4 or 8 KB apart, the other kernels'
